@@ -14,9 +14,9 @@
 //  * dense_gemv2_kernel (n <= 8 while the token tile's activations fit 64 KB of LDS; HBM-bound): activations
 //    staged in LDS, each wave streaming 1..4 rows two 16-byte pieces per lane deep; dense_gemv_kernel
 //    otherwise: a wave streams 8 rows with 16-byte loads, the activations from L2.
-//  * dense_mfma_kernel (n > 8): each wave owns 32 rows x 64 tokens on the matrix cores, its A and B fragments
-//    loaded straight from global memory: v_mfma_f32_32x32x16_bf16 on bf16-rounded activations, else
-//    v_mfma_f32_32x32x2_f32 on exact f32 operands.
+//  * dense_tile_kernel (F32, and BF16 with unrounded activations, past the GEMV): v_mfma_f32_*f32 on exact operands loaded
+//    straight from global memory, one tile per workgroup, its waves splitting k.
+//  * dense_mma_kernel (F16, and BF16 with rounded activations, past the GEMV): LDS-staged f16 / bf16 matrix cores.
 #include "common.h"
 #include "launch.h"
 
@@ -130,9 +130,12 @@ __global__ void __launch_bounds__(64 * DG_WAVES) dense_gemv_kernel(WeightView w,
 // is multiplied. The loads are unconditional (a step past the row's end re-reads the last piece and adds
 // nothing), so the compiler waits for exactly the step it computes. Columns past k inside a row's last
 // piece are zeroed before use (a pinned row's may hold anything, NaN included).
-constexpr int DG2_LDS_MAX = 64 * 1024;
+constexpr int DG2_LDS_MAX = 64 * 1024, DG2_KSPLIT_ROWS = 256;
 
-template <int DT, int NT, int RPW>
+// KS (one row per workgroup): the four waves take every fourth step of the row instead of a row each, and their sums
+// meet in LDS. A router of 32 rows is 8 workgroups walking 12 dependent steps otherwise (F32 32x2880, one token:
+// 4.5 -> 3.5 us, 256x4096: 7.0 -> 4.7, F16 256x4096: 5.6 -> 4.2).
+template <int DT, int NT, int RPW, bool KS = false>
 __global__ void __launch_bounds__(64 * DG_WAVES) dense_gemv2_kernel(WeightView w, const float* __restrict__ a, int lda,
                                                                     int k, int m, int n, float* __restrict__ c,
                                                                     int ldc, int rnd, int kp, Epi ep) {
@@ -140,8 +143,10 @@ __global__ void __launch_bounds__(64 * DG_WAVES) dense_gemv2_kernel(WeightView w
     extern __shared__ __align__(16) float xs[];   // [NT][kp], kp a multiple of 64·V
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int t0 = blockIdx.y * NT, ntv = n - t0 < NT ? n - t0 : NT;
-    const int64_t row0 = ((int64_t) blockIdx.x * DG_WAVES + wave) * RPW;
-    const int S = kp / (64 * V);                  // steps per row
+    const int64_t row0 = KS ? (int64_t) blockIdx.x : ((int64_t) blockIdx.x * DG_WAVES + wave) * RPW;
+    static_assert(!KS || RPW == 1, "a split row is alone in its workgroup");
+    constexpr int JS = KS ? DG_WAVES : 1;         // step stride of a wave
+    const int S = kp / (64 * V), jw = KS ? wave : 0;   // steps per row, the wave's first one
     const uint8_t* wr[RPW];
 #pragma unroll
     for (int r = 0; r < RPW; r++) {
@@ -156,8 +161,8 @@ __global__ void __launch_bounds__(64 * DG_WAVES) dense_gemv2_kernel(WeightView w
         for (int r = 0; r < RPW; r++) raw[r] = ld16_nt(wr[r] + (int64_t) e0 * ES);
     };
     uint4 raw[2][RPW];
-    load(raw[0], 0);
-    load(raw[1], 1);
+    load(raw[0], jw);
+    load(raw[1], jw + JS);
     // stage the tile's activations: float4 slots of [NT][kp]
     const int q4 = kp / 4;
     for (int i = threadIdx.x; i < NT * q4; i += 64 * DG_WAVES) {
@@ -203,11 +208,26 @@ __global__ void __launch_bounds__(64 * DG_WAVES) dense_gemv2_kernel(WeightView w
                 for (int i = 0; i < V; i++) acc[r][t] = fmaf(f[r][i], x[i], acc[r][t]);
         }
     };
-    for (int j = 0; j < S; j += 2) {
+    for (int j = jw; j < S; j += 2 * JS) {
         step(raw[0], j);
-        load(raw[0], j + 2);
-        if (j + 1 < S) step(raw[1], j + 1);
-        load(raw[1], j + 3);
+        load(raw[0], j + 2 * JS);
+        if (j + JS < S) step(raw[1], j + JS);
+        load(raw[1], j + 3 * JS);
+    }
+    if constexpr (KS) {   // every wave reaches this: row0 < m for the whole workgroup
+        __shared__ float part[DG_WAVES][NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const float v = wave_sum(acc[0][t]);
+            if (lane == 0) part[wave][t] = v;
+        }
+        __syncthreads();
+        if ((int) threadIdx.x < ntv) {
+            const int t = threadIdx.x;
+            float* dst = c + (int64_t) (t0 + t) * ldc + row0;
+            *dst = epilogue(ep, (part[0][t] + part[1][t]) + (part[2][t] + part[3][t]), row0, dst);
+        }
+        return;
     }
 #pragma unroll
     for (int r = 0; r < RPW; r++)
@@ -223,81 +243,103 @@ __global__ void __launch_bounds__(64 * DG_WAVES) dense_gemv2_kernel(WeightView w
 }
 
 // ------------------------------------------------------------------------------------------ GEMM
-// Wave tile: 32 rows x 64 tokens (two 32x32 accumulators sharing the A fragment). Lane (r, q) = (lane % 32,
-// lane / 32) loads row r's and token r's operands for the K positions the instruction assigns to q; the
-// accumulator holds token r, rows 8·(e / 4) + 4q + e % 4.
-constexpr int DM_WAVES = 4;
+// F32 weights, and BF16 weights with unrounded activations (n > 8, or past the GEMV's LDS): f32 MFMA on exact operands.
+// One wave per 32 x 64 tile, walking k alone behind its own loads, held 32 rows x 512 tokens (a router) to 8 waves on
+// 2 CUs: 296 us at k = 2880. Here a workgroup of 8 waves owns one T x T tile (16 or 32) and its waves take every
+// eighth run of k: 64 CUs on that shape, 12.3 us (2.7 us of it the f32 matrix rate of one CU on a 16 x 16 x 2880 tile), and
+// more than twice as fast where the tiles fill the chip (F32 4096x4096 n = 512: 556 -> 255 us; 2048x2880 n = 512:
+// 391 -> 95). Two or three runs in flight per wave instead of one lose 5 to 30%: the registers cost more waves than the
+// distance hides. The waves' sums meet in LDS in a fixed order.
+// 32 x 32 tiles halve the bytes read per product and take over once they give most CUs one (F32 512x2880 n = 512, 256 such
+// tiles: 25 against 50.8 us; 1024x2880 n = 128, 128 tiles, stays with 16 x 16: 24.4 us).
+constexpr int64_t DENSE_TILE32_MIN = 192;
+constexpr int DT_WAVES = 8;
 
-template <int DT, bool BF16MMA>
-__global__ void __launch_bounds__(64 * DM_WAVES) dense_mfma_kernel(WeightView w, const float* __restrict__ a, int lda,
+template <int DT, int T>
+__global__ void __launch_bounds__(64 * DT_WAVES) dense_tile_kernel(WeightView w, const float* __restrict__ a, int lda,
                                                                    int k, int m, int n, float* __restrict__ c, int ldc,
-                                                                   Epi ep) {
+                                                                   int nt, int vec, Epi ep) {
+    constexpr int Q = 64 / T, RUN = 16 * Q, E = T * T / 64, LD = T + 4;
     constexpr int ES = block_bytes(DT);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, q = lane >> 5;
-    const int64_t row0 = ((int64_t) blockIdx.x * DM_WAVES + wave) * 32;
-    if (row0 >= m) return;   // wave-uniform; no barrier
-    const int t0 = blockIdx.y * 64;
-    const int64_t wrow = row0 + r < m ? row0 + r : m - 1;
+    static_assert(DT == F32 || DT == BF16, "F16 takes the staged GEMM");
+    typedef float accv __attribute__((ext_vector_type(E)));
+    __shared__ __align__(16) float red[DT_WAVES][T * LD];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane % T, q = lane / T;
+    const int64_t row0 = (int64_t) (blockIdx.x / nt) * T;   // nt token tiles per row tile
+    const int t0 = (int) (blockIdx.x % nt) * T;
+    const int64_t wrow = row0 + r < m ? row0 + r : m - 1;   // clamped: its products are never stored
+    const int trow = t0 + r < n ? t0 + r : n - 1;
     const uint8_t* wp = w.qs + (w.r0 + wrow) * w.G;
-    const int tA = t0 + r, tB = t0 + 32 + r;
-    const float* aA = a + (int64_t) (tA < n ? tA : n - 1) * lda;
-    const float* aB = a + (int64_t) (tB < n ? tB : n - 1) * lda;
-    const bool vA = tA < n, vB = tB < n;
-    floatx16 accA = floatx16{}, accB = floatx16{};
-    if constexpr (BF16MMA) {
-        // one 32x32x16 step: lane (r, q) holds K positions 8q .. 8q + 7 of the step
-        for (int k0 = 0; k0 < k; k0 += 16) {
-            const int kb = k0 + 8 * q;
-            uint4 wv = kb < k ? *reinterpret_cast<const uint4*>(wp + (int64_t) kb * ES) : make_uint4(0, 0, 0, 0);
-            if (kb + 8 > k) {   // the row's last piece: columns past k (a pinned row's may hold anything) -> 0
-                uint32_t u[4] = {wv.x, wv.y, wv.z, wv.w};
+    const float* ap = a + (int64_t) trow * lda;
+    const int runs = (k + RUN - 1) / RUN;
+    // Piece i of a run is 4·Q consecutive k of a row, 4 per lane, so a load instruction reads 16·Q (F32) contiguous bytes
+    // of T rows. A run never crosses a row's 256-byte pitch (RUN·ES divides it): weight loads past k stay in the row.
+    typedef uint32_t piece __attribute__((ext_vector_type(ES)));   // 4 weights
+    auto load = [&](piece (&wv)[4], float4 (&xv)[4], int it) {
+        const int e0 = it * RUN + 4 * q;
 #pragma unroll
-                for (int i = 0; i < 8; i++)
-                    if (kb + i >= k) u[i >> 1] &= (i & 1) ? 0x0000ffffu : 0xffff0000u;
-                wv = make_uint4(u[0], u[1], u[2], u[3]);
-            }
-            const bf16x8 A = __builtin_bit_cast(bf16x8, wv);
-            uint32_t ba[4], bb[4];
+        for (int i = 0; i < 4; i++) wv[i] = *reinterpret_cast<const piece*>(wp + (int64_t) (e0 + 4 * Q * i) * ES);
+        if (vec && (it + 1) * RUN <= k) {   // wave-uniform
+#pragma unroll
+            for (int i = 0; i < 4; i++) xv[i] = *reinterpret_cast<const float4*>(ap + e0 + 4 * Q * i);
+        } else {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int kk = kb + 2 * i;
-                const uint32_t a0 = bf16_bits(kk < k && vA ? aA[kk] : 0.0f), a1 = bf16_bits(kk + 1 < k && vA ? aA[kk + 1] : 0.0f);
-                const uint32_t b0 = bf16_bits(kk < k && vB ? aB[kk] : 0.0f), b1 = bf16_bits(kk + 1 < k && vB ? aB[kk + 1] : 0.0f);
-                ba[i] = a0 | (a1 << 16);
-                bb[i] = b0 | (b1 << 16);
+                const int e = e0 + 4 * Q * i;
+                xv[i] = make_float4(e < k ? ap[e] : 0.0f, e + 1 < k ? ap[e + 1] : 0.0f, e + 2 < k ? ap[e + 2] : 0.0f,
+                                    e + 3 < k ? ap[e + 3] : 0.0f);
             }
-            const bf16x8 BA = __builtin_bit_cast(bf16x8, make_uint4(ba[0], ba[1], ba[2], ba[3]));
-            const bf16x8 BB = __builtin_bit_cast(bf16x8, make_uint4(bb[0], bb[1], bb[2], bb[3]));
-            accA = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, BA, accA, 0, 0, 0);
-            accB = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, BB, accB, 0, 0, 0);
         }
-    } else {
-        // four 32x32x2 steps per 8 K positions: lane (r, q) loads positions 4q .. 4q + 3, step j takes the j-th
-        for (int k0 = 0; k0 < k; k0 += 8) {
-            const int kb = k0 + 4 * q;
-            float wf[4];
+    };
+    accv acc[2] = {accv{}, accv{}};
+    auto mul = [&](const piece (&wv)[4], const float4 (&xv)[4], int it) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float f[4];
             if constexpr (DT == F32) {
-                const uint4 v = kb < k ? *reinterpret_cast<const uint4*>(wp + (int64_t) kb * 4) : make_uint4(0, 0, 0, 0);
-                wvals<F32>(v, wf);
+#pragma unroll
+                for (int u = 0; u < 4; u++) f[u] = __builtin_bit_cast(float, (uint32_t) wv[i][u]);
             } else {
-                const uint2 v = kb < k ? *reinterpret_cast<const uint2*>(wp + (int64_t) kb * 2) : make_uint2(0, 0);
-                float f8[8];
-                wvals<DT>(make_uint4(v.x, v.y, 0u, 0u), f8);
 #pragma unroll
-                for (int i = 0; i < 4; i++) wf[i] = f8[i];
+                for (int u = 0; u < 4; u++)
+                    f[u] = __builtin_bit_cast(float, u & 1 ? wv[i][u / 2] & 0xffff0000u : wv[i][u / 2] << 16);
             }
+            if ((it + 1) * RUN > k) {   // a pinned row's columns past k may hold anything
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int kk = kb + j;
-                wf[j] = kk < k ? wf[j] : 0.0f;   // columns past k (a pinned row's may hold anything) -> 0
-                const float xa = kk < k && vA ? aA[kk] : 0.0f, xb = kk < k && vB ? aB[kk] : 0.0f;
-                accA = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[j], xa, accA, 0, 0, 0);
-                accB = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[j], xb, accB, 0, 0, 0);
+                for (int u = 0; u < 4; u++) f[u] = it * RUN + 4 * q + 4 * Q * i + u < k ? f[u] : 0.0f;
+            }
+            const float x[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                if constexpr (T == 16)
+                    acc[u & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[u], x[u], acc[u & 1], 0, 0, 0);
+                else
+                    acc[u & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(f[u], x[u], acc[u & 1], 0, 0, 0);
             }
         }
+    };
+    for (int it = wave; it < runs; it += DT_WAVES) {
+        piece wv[4];
+        float4 xv[4];
+        load(wv, xv, it);
+        mul(wv, xv, it);
     }
-    if (vA) store_column(c + (int64_t) tA * ldc, row0 + 4 * q, m, accA, 1.0f, ep, false);
-    if (vB) store_column(c + (int64_t) tB * ldc, row0 + 4 * q, m, accB, 1.0f, ep, false);
+    // lane: token r, rows 4q + e (T = 16) or 8·(e / 4) + 4q + e % 4 (T = 32)
+    const accv s = acc[0] + acc[1];
+#pragma unroll
+    for (int g = 0; g < E / 4; g++)
+        *reinterpret_cast<float4*>(&red[wave][r * LD + 8 * g + 4 * q]) =
+            make_float4(s[4 * g], s[4 * g + 1], s[4 * g + 2], s[4 * g + 3]);
+    __syncthreads();
+    for (int i = threadIdx.x; i < T * T; i += 64 * DT_WAVES) {
+        const int row = i % T, t = i / T;
+        if (row0 + row >= m || t0 + t >= n) continue;
+        float v = red[0][t * LD + row];
+#pragma unroll
+        for (int u = 1; u < DT_WAVES; u++) v += red[u][t * LD + row];
+        float* dst = c + (int64_t) (t0 + t) * ldc + row0 + row;
+        *dst = epilogue(ep, v, row0 + row, dst);
+    }
 }
 
 // ------------------------------------------------------------------------- staged matrix-core GEMM (n >= 9)
@@ -488,13 +530,19 @@ __global__ void __launch_bounds__(256, 2) dense_mma_kernel(WeightView w, const u
 // jam rounds BF16's activations to bf16 where its bf16 kernels take the call (jam.c:622-652).
 static bool bf16_rounds(int n, int k) { return (n >= 8 && k % 2 == 0) || k % 32 == 0; }
 
-template <int DT, int NT, int RPW>
+template <int DT, int NT, int RPW, bool KS = false>
 static void gemv2_go(const WeightView& w, const float* a, int lda, int k, int kp, int m, int n, float* c, int ldc,
                      int rnd, hipStream_t st, const Epi& ep) {
-    const int rows_per_wg = DG_WAVES * RPW;
+    const int rows_per_wg = KS ? 1 : DG_WAVES * RPW;
     const dim3 grid((unsigned) ((m + rows_per_wg - 1) / rows_per_wg), (unsigned) ((n + NT - 1) / NT));
-    dense_gemv2_kernel<DT, NT, RPW><<<grid, 64 * DG_WAVES, (size_t) NT * kp * 4, st>>>(w, a, lda, k, m, n, c, ldc, rnd,
+    dense_gemv2_kernel<DT, NT, RPW, KS><<<grid, 64 * DG_WAVES, (size_t) NT * kp * 4, st>>>(w, a, lda, k, m, n, c, ldc, rnd,
                                                                                        kp, ep);
+}
+
+// The NT-token tile of n <= 8 tokens fits the staged GEMV's LDS.
+static bool gemv2_fits(int n, int dt, int k) {
+    const int nt = n <= 2 ? n : n <= 4 ? 4 : 8, run = 64 * 16 / block_bytes(dt), kp = (k + run - 1) / run * run;
+    return (size_t) nt * kp * 4 <= (size_t) DG2_LDS_MAX;
 }
 
 template <int DT, int NT>
@@ -503,36 +551,45 @@ static void gemv_go(const WeightView& w, const float* a, int lda, int k, int m, 
     constexpr int V = 16 / block_bytes(DT);
     const int kp = (k + 64 * V - 1) / (64 * V) * (64 * V);
     if ((size_t) NT * kp * 4 <= (size_t) DG2_LDS_MAX) {
+        // up to a row per CU: a workgroup per row, its waves splitting k (four times as many workgroups; from there
+        // on the one-row waves alone fill the CUs)
+        if (m <= DG2_KSPLIT_ROWS) return gemv2_go<DT, NT, 1, true>(w, a, lda, k, kp, m, n, c, ldc, rnd, st, ep);
         // rows per wave: about 2048 waves or more over the device, 4 rows a wave at most
         if (m >= 4 * 2048) return gemv2_go<DT, NT, 4>(w, a, lda, k, kp, m, n, c, ldc, rnd, st, ep);
         if (m >= 2 * 2048) return gemv2_go<DT, NT, 2>(w, a, lda, k, kp, m, n, c, ldc, rnd, st, ep);
         return gemv2_go<DT, NT, 1>(w, a, lda, k, kp, m, n, c, ldc, rnd, st, ep);
     }
-    const int rows_per_wg = DG_WAVES * DG_RPW;
+    const int rows_per_wg = DG_WAVES * DG_RPW;   // one token, k past the staged GEMV's LDS
     const dim3 grid((unsigned) ((m + rows_per_wg - 1) / rows_per_wg), (unsigned) ((n + NT - 1) / NT));
-    dense_gemv_kernel<DT, NT><<<grid, 64 * DG_WAVES, 0, st>>>(w, a, lda, k, m, n, c, ldc, rnd, ep);
+    if constexpr (NT == 1) dense_gemv_kernel<DT, NT><<<grid, 64 * DG_WAVES, 0, st>>>(w, a, lda, k, m, n, c, ldc, rnd, ep);
 }
 
 template <int DT>
 static hipError_t dense_go(const WeightView& w, const float* a, int lda, int k, int m, int n, float* c, int ldc,
                            hipStream_t st, const Epi& ep) {
     const bool rnd = DT == BF16 && bf16_rounds(n, k);
-    if (n <= 8) {
+    if (n == 1 || (n <= 8 && gemv2_fits(n, DT, k))) {
         if (n == 1) gemv_go<DT, 1>(w, a, lda, k, m, n, c, ldc, rnd, st, ep);
         else if (n == 2) gemv_go<DT, 2>(w, a, lda, k, m, n, c, ldc, rnd, st, ep);
         else if (n <= 4) gemv_go<DT, 4>(w, a, lda, k, m, n, c, ldc, rnd, st, ep);
         else gemv_go<DT, 8>(w, a, lda, k, m, n, c, ldc, rnd, st, ep);
         return hipGetLastError();
     }
-    const dim3 grid((unsigned) ((m + 32 * DM_WAVES - 1) / (32 * DM_WAVES)), (unsigned) ((n + 63) / 64));
-    if constexpr (DT == BF16) {
-        if (rnd) {
-            dense_mfma_kernel<DT, true><<<grid, 64 * DM_WAVES, 0, st>>>(w, a, lda, k, m, n, c, ldc, ep);
-            return hipGetLastError();
-        }
+    // F16 and bf16-rounded BF16 calls of 2 or more tokens past the GEMV took the staged GEMM (dense_mma_planes)
+    if constexpr (DT != F16) {
+        const int vec = lda % 4 == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0;
+        const int64_t nt32 = (n + 31) / 32, tiles32 = (int64_t) ((m + 31) / 32) * nt32;
+        const int64_t nt16 = (n + 15) / 16, tiles16 = (int64_t) ((m + 15) / 16) * nt16;
+        if (tiles32 > 0x7fffffff) return hipErrorInvalidValue;
+        if (tiles32 >= DENSE_TILE32_MIN)
+            dense_tile_kernel<DT, 32><<<(unsigned) tiles32, 64 * DT_WAVES, 0, st>>>(w, a, lda, k, m, n, c, ldc, (int) nt32,
+                                                                                    vec, ep);
+        else
+            dense_tile_kernel<DT, 16><<<(unsigned) tiles16, 64 * DT_WAVES, 0, st>>>(w, a, lda, k, m, n, c, ldc, (int) nt16,
+                                                                                    vec, ep);
+        return hipGetLastError();
     }
-    dense_mfma_kernel<DT, false><<<grid, 64 * DM_WAVES, 0, st>>>(w, a, lda, k, m, n, c, ldc, ep);
-    return hipGetLastError();
+    return hipErrorInvalidValue;
 }
 
 // 2 planes (F16: hi, lo), 1 (BF16 with jam's bf16 rounding), 0: the staged GEMM does not take the call. It
@@ -543,8 +600,7 @@ int dense_mma_planes(int dt, int n, int k) {
     if (dt != F16 && !(dt == BF16 && bf16_rounds(n, k))) return 0;
     if (n < DENSE_MMA_MIN_N) {
         if (n < 2) return 0;
-        const int nt = n == 2 ? 2 : n <= 4 ? 4 : 8, kp = (k + 64 * 8 - 1) / (64 * 8) * (64 * 8);
-        if ((size_t) nt * kp * 4 <= (size_t) DG2_LDS_MAX) return 0;
+        if (gemv2_fits(n, dt, k)) return 0;
     }
     return dt == F16 ? 2 : 1;
 }
