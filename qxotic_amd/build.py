@@ -39,6 +39,7 @@ UNITS = {   # source -> extra flags
     "dense.hip": [],
     "gemm.hip": [],
     "mma.hip": [],
+    "mx4.hip": [],
     "mxn.hip": [],
     "moe.hip": ["-ffp-contract=off"],
     "epilogue.hip": ["-ffp-contract=off"],

@@ -30,8 +30,7 @@ __host__ __device__ constexpr bool is_dense(int dt) { return dt == F32 || dt == 
 //   Q6_K : NC 13 chunks 0-7 ql, 8-11 qh, 12 the 16 int8 scales | SB 2 : d fp16
 //   Q8_0 : NC 16 chunk c = half c&1 of block c>>1 (int8 q)     | SB 16: the 8 blocks' fp16 d
 //   Q4_0 : NC 8  chunk c = block c's 16 nibble bytes           | SB 16: the 8 blocks' fp16 d
-//   MXFP4: NC 8  chunk c = block c's 16 nibble bytes           | SB 16: the 8 blocks' e8m0, then their
-//                                                                maximum (the group's reference exponent)
+//   MXFP4: NC 8  chunk c = block c's 16 nibble bytes           | SB 16: the 8 blocks' e8m0, then their maximum
 //   Q5_K : NC 10 chunks 0-7 qs nibble bytes, 8-9 the qh bytes   | SB 16: d, dmin, 12 scale bytes
 //   NVFP4: NC 8  chunk 2j + h = half h of 64-block j's qs       | SB 16: the 4 blocks' 4 UE4M3 scales
 //   Q1_0 : NC 2  chunk j = 128-block j's 16 sign bytes          | SB 4 : the 2 blocks' fp16 d
@@ -127,6 +126,10 @@ __device__ inline void store_column(float* ct, int64_t rowb, int64_t m, const V&
         }
     }
 }
+
+// Largest MXFP4 block exponent of the matrix-core kernel: its exact block sums 2^(e - 128)·Σ kv·q, below 2^(e - 111), stay
+// finite (mx4.hip).
+constexpr int MX4_MAX_E = 238;
 
 struct WeightView {
     const uint8_t* qs;   // plane 0 of the device copy

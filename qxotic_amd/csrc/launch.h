@@ -15,8 +15,8 @@ hipError_t launch_quant_f1(const float* a, int lda, int n, int k, int8_t* q, flo
 hipError_t launch_quant_f2(const float* a, int lda, int n, int k, int8_t* q, float* d, float* xs, hipStream_t st);
 
 // raw GGUF rows (rb blocks each, stride raw_stride bytes) -> the device layout with G groups per row. For
-// Q8_0, Q4_0 and MXFP4 with a non-null flag (device int), *flag ends 1 if some group's block scales cannot
-// be folded exactly into the matrix-core GEMM's f16 operands (prep.hip, repack_kernel), else 0.
+// Q8_0, Q4_0 and MXFP4 with a non-null flag (device int), *flag ends 1 if some group's block scales keep the tensor
+// off the matrix-core GEMMs (prep.hip, repack_kernel), else 0.
 hipError_t launch_repack(int dt, const uint8_t* raw, int64_t raw_stride, int64_t rows, int64_t rb, int64_t G,
                          uint8_t* qs, uint8_t* sc, hipStream_t st, int* flag = nullptr);
 
@@ -123,6 +123,9 @@ struct GemmAct {
     const _Float16* shi;   // per-32 sums (Q4_K, Q4_0) [Kp/256][NP][8] or per-16 sums (Q6_K) [Kp/256][NP][16],
     const _Float16* slo;   //   · 2^-e_t, split as f16 high part + f16 remainder
     const float* es;       // [NP] 2^e_t
+    // MXFP4 (mx4.hip): b holds the first 16 bytes and b8 the last 8 of each block's 32 high (0) or low (1) digits, 6
+    // bits each in the order of the weights' nibbles, [Kp/32][2][NP][16 B] and [..][8 B]; dx is [Kp/128][NP][4]
+    const uint8_t* b8;
     int NP, Kp;
     int K;                 // the call's k (blocks past it are zero)
 };
@@ -149,6 +152,10 @@ hipError_t launch_gemm_mma(int dt, const WeightView& w, const GemmAct& A, int k,
 hipError_t launch_gemm_mma_grouped(int dt, const WeightView& w, const GemmAct& A, int k, const Groups& g, int cap64,
                                    float* c, int ldc, hipStream_t st);
 size_t gemm_act_bytes_np(int dt, int NP, int k);
+// The MXFP4 kernel behind both (mx4.hip): rt row tiles per wave, ns K slices of sb_per super-blocks writing partials
+// c_slice floats apart (0: none), the last xsplit tiles of each XCD's run as half tiles.
+hipError_t launch_mx4_gemm(const WeightView& w, const GemmAct& A, int m, int n, float* c, int ldc, hipStream_t st,
+                           const Groups& gp, int rt, int ns, int sb_per, int xsplit, int64_t c_slice, const Epi& ep);
 
 // Opt-in native-MX path for MXFP4 (mxn.hip): activations as MX-FP8 hi + lo codes (mode 1) or hi only
 // (mode 2) in the scaled MFMA's B operand order, one e8m0 scale per 32-block for each part.

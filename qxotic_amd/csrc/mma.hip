@@ -1,4 +1,4 @@
-// Matrix-core prefill GEMM for Q4_K, Q5_K, Q6_K, MXFP4, Q4_0 and Q8_0 weights: C[n][m] = W[m][k] · A[n][k]^T with jam's
+// Matrix-core prefill GEMM for Q4_K, Q5_K, Q6_K, Q4_0, Q8_0, NVFP4 and Q1_0 weights (MXFP4: mx4.hip): C[n][m] = W[m][k] · A[n][k]^T with jam's
 // F2 semantics (the n >= 8 bands of jam_kernels_q4k_avx512.c), activations from launch_gemm_prep.
 //
 // Arithmetic. Each 32-element block's integer dot runs on v_mfma_f32_32x32x16_f16 with integer operands
@@ -19,8 +19,7 @@
 // Operands. With the 32-row tiles of the device layout, the A fragment of lane (r, q) (row r = lane % 32,
 // q = lane / 32) for K-step ks of a block is the low or high nibbles of bytes 8ks..8ks+7 of one 16-byte
 // chunk, turned into f16 pairs from bytes (0,2), (1,3), (4,6), (5,7) by mask-and-or with 0x6400 (1024 + v)
-// and one packed FMA with the scale (which removes the 1024). MXFP4 instead converts each byte's two nibbles
-// (elements e, e + 16) with the hardware e2m1 conversion. The activation codes are stored in the matching
+// and one packed FMA with the scale (which removes the 1024). The activation codes are stored in the matching
 // order (GemmAct::b), so no shuffle is needed on either side.
 //
 // Tiling. A workgroup of 4 waves owns 4·RT row tiles (32 rows each, wave w the RT tiles w·RT..) x CT token
@@ -106,19 +105,6 @@ JAMHIP_DEV uint32_t word(const uint4& v, int i) { return i == 0 ? v.x : i == 1 ?
 
 JAMHIP_DEV float h2f_bits(uint32_t b) { return (float) __builtin_bit_cast(_Float16, (uint16_t) (b & 0xffffu)); }
 
-// MXFP4: 8 f16 of one K-step from one word (4 bytes) of a block's nibble bytes, by the hardware e2m1
-// conversion: byte u gives the pair (e2m1(low nibble), e2m1(high nibble))·scale, elements e and e + 16 of the
-// block (the activation codes are stored in the same order, GemmAct). scale = 2^(e_block − e_ref + 1) turns
-// e2m1 into jam's doubled value x2 (jam_mxfp4.h:14-15: 0,1,2,3,4,6,8,12) times 2^(e_block − e_ref).
-JAMHIP_DEV half8 mx_frag(uint32_t w, float scale) {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    const h2 p0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 0);
-    const h2 p1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 1);
-    const h2 p2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 2);
-    const h2 p3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 3);
-    return half8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-}
-
 // Q1_0: 8 f16 of one K-step from one byte of sign bits, bit j = element j of the run, each as 2^-14 (the
 // smallest normal f16, bit 10) or 0, in the frag8 pair order (bits 0,2), (1,3), (4,6), (5,7): with x = B | B << 14
 // bit j sits at j and j + 14, so x << (10 - j0) puts bits j0 and j0 + 2 at bits 10 and 26.
@@ -195,7 +181,7 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) kq_gemm_kernel(WeightView w, G
     // split K (sb_per > 0): slice blockIdx.y takes super-blocks [sb_per·y, sb_per·(y + 1)) and writes its
     // partial result to c + y·c_slice (summed by split_reduce_kernel); stages are half super-blocks
     const int st0 = sb_per > 0 ? 2 * sb_per * (int) blockIdx.y : 0;
-    // stages that hold at least one block of k (MXFP4 pads k to whole groups: k = 2880 needs 23 of 24)
+    // stages that hold at least one block of k (k is padded to whole groups: Q8_0 at k = 2880 needs 23 of 24)
     const int nstk = min(2 * nsb, (A.K / 32 + 3) / 4);
     const int nst = sb_per > 0 ? min(nstk, st0 + 2 * sb_per) : nstk;
     int64_t r0t = w.r0 >> 5;                     // the view's first row is tile-aligned (launcher checks)
@@ -224,7 +210,7 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) kq_gemm_kernel(WeightView w, G
     const int64_t Tw = T0 + wave < tiles ? T0 + wave : tiles - 1;             // this wave's row tile
     const uint8_t* a_src = w.qs + (r0t + Tw) * G * (NC * CHUNK_STRIDE) + 16 * lane;
     const int a_dst = S::A_OFF + wave * NCS * 512;
-    // headers: Q4_K / MXFP4 16 B per row, tiles 2·wave + q (waves 0, 1); Q6_K d, 8 rows per lane (wave 0)
+    // headers: Q4_K and others 16 B per row, tiles 2·wave + q (waves 0, 1); Q6_K d, 8 rows per lane (wave 0)
     const uint8_t* h_src;
     if constexpr (DT == Q1_0) {   // 4 B per row: lanes 0..31 of wave 0 copy 16 B each, tile lane / 8
         const int64_t T = T0 + (lane >> 3) < tiles ? T0 + (lane >> 3) : tiles - 1;
@@ -254,7 +240,7 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) kq_gemm_kernel(WeightView w, G
 #pragma unroll
             for (int p = 0; p < 2; p++) dma16(ag + (4 * h2 + 2 * p) * CHUNK_STRIDE, buf + a_dst + 2 * p * 512);
             dma16(ag + 8 * CHUNK_STRIDE, buf + a_dst + 4 * 512);
-        } else if constexpr (DT != Q6_K) {   // Q4_K chunks 4h2..4h2+3 (sub-block pairs), MXFP4 / Q4_0 blocks
+        } else if constexpr (DT != Q6_K) {   // Q4_K chunks 4h2..4h2+3 (sub-block pairs), Q4_0 blocks
                                              // 4h2..4h2+3, Q8_0 chunks 8h2..8h2+7 (two per block)
 #pragma unroll
             for (int p = 0; p < NCS / 2; p++)
@@ -591,88 +577,6 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) kq_gemm_kernel(WeightView w, G
                             accs[i][j] = floatx16{};
                         }
                     }
-                }
-            } else if constexpr (DT == MXFP4) {   // group of 8 blocks; stage h2 = blocks 4h2..4h2+3
-                // every LDS read of the stage up front, then the next stage's copy, then the compute
-                uint4 hdr[RT];
-                uint2 chs[RT][4];   // lane half q: bytes 8q..8q+7 of each block (K-step 0 word 2q, K-step 1 word 2q + 1)
-                half8 bfs[4][CT][2];
-                float dxs[4][CT];
-                float sg[RT][16];
-    #pragma unroll
-                for (int i = 0; i < RT; i++) {
-                    hdr[i] = *reinterpret_cast<const uint4*>(buf + S::H_OFF + ((wave * RT + i) * 32 + r) * 16);
-    #pragma unroll
-                    for (int bl = 0; bl < 4; bl++)
-                        chs[i][bl] = *reinterpret_cast<const uint2*>(LA + ((wave * RT + i) * NCS + bl) * 512 + 16 * r + 8 * q);
-                }
-    #pragma unroll
-                for (int bl = 0; bl < 4; bl++)
-    #pragma unroll
-                    for (int j = 0; j < CA; j++) {
-    #pragma unroll
-                        for (int ks = 0; ks < 2; ks++)
-                            bfs[bl][j][ks] = *reinterpret_cast<const half8*>(LB + ((2 * bl + ks) * 2 + q) * BN * 16 + (32 * j + r) * 16);
-                        dxs[bl][j] = LDX[bl * BN + 32 * j + r];
-                    }
-                const bool gend = h2 == 1 || st == nstk - 1;   // the last group may end after its first half
-                if (gend) {   // group end: 2^(e_ref - 128) of the 16 output rows this lane holds (header bytes 12..15)
-    #pragma unroll
-                    for (int i = 0; i < RT; i++) {
-                        const unsigned char* H = buf + S::H_OFF + (wave * RT + i) * 32 * 16 + 12;
-    #pragma unroll
-                        for (int e = 0; e < 16; e++)
-                            sg[i][e] = *reinterpret_cast<const float*>(H + (8 * (e >> 2) + 4 * q + (e & 3)) * 16);
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                if (st + 1 < nst) issue(st + 1, smem + ((st + 1) & 1) * S::BYTES);
-                // software pipeline: block bl's products go out before block bl-1's scale FMAs
-                floatx16 Dp[2][RT][CT];
-    #pragma unroll
-                for (int bl = 0; bl < 5; bl++) {
-                    if (bl < 4) {
-                        half8 af[RT][2];
-    #pragma unroll
-                        for (int i = 0; i < RT; i++) {
-                            const uint2 ch = chs[i][bl];
-                            const int eb = (int) (((h2 ? hdr[i].y : hdr[i].x) >> (8 * bl)) & 0xffu);
-                            const int er = (int) (hdr[i].z & 0xffu);
-                            // f32 bits of 2^(eb - er + 1): (eb - er)·2^23 + bits(2.0); a scale below 2^-126 (only a
-                            // zero-code block stored as e = 0 under a reference >= 128) comes out <= 0 and becomes 0
-                            const int sb = (eb - er) * (1 << 23) + 0x40000000;
-                            const float scale = __builtin_bit_cast(float, max(sb, 0));
-                            af[i][0] = mx_frag(ch.x, scale);
-                            af[i][1] = mx_frag(ch.y, scale);
-                        }
-    #pragma unroll
-                        for (int i = 0; i < RT; i++)
-    #pragma unroll
-                            for (int j = 0; j < CA; j++) {
-                                floatx16 D = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i][0], bfs[bl][j][0], floatx16{}, 0, 0, 0);
-                                Dp[bl & 1][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i][1], bfs[bl][j][1], D, 0, 0, 0);
-                            }
-                    }
-                    if (bl > 0) {
-                        const int pb = bl - 1;
-    #pragma unroll
-                        for (int i = 0; i < RT; i++)
-    #pragma unroll
-                            for (int j = 0; j < CA; j++)
-    #pragma unroll
-                                for (int e = 0; e < 16; e++)
-                                    accs[i][j][e] = fmaf(Dp[pb & 1][i][j][e], dxs[pb][j], accs[i][j][e]);
-                    }
-                }
-                if (gend) {   // group end: acc += 2^(e_ref - 128) · accs
-    #pragma unroll
-                    for (int i = 0; i < RT; i++)
-    #pragma unroll
-                        for (int j = 0; j < CA; j++) {
-    #pragma unroll
-                            for (int e = 0; e < 16; e++) acc[i][j][e] = fmaf(sg[i][e], accs[i][j][e], acc[i][j][e]);
-                            accs[i][j] = floatx16{};
-                        }
                 }
             } else if constexpr (DT == Q1_0) {
                 // stage h2 = 128-block h2 of the group (one chunk of sign bits, d = the row's fp16 d[h2]). jam's F2
@@ -1044,6 +948,25 @@ static hipError_t kq_go(const WeightView& w, const GemmAct& A, int m, int n, flo
     return hipGetLastError();
 }
 
+// MXFP4 (mx4.hip): waves of 64 rows (256-row workgroups, k whole) once those give each CU one, or at k <= 4096, where a
+// whole k is short, once they give every third CU one; else waves of 32 rows with the K split of the other types.
+// 64 against 32 rows: 14336x4096 n = 320 55.7 / 67.2 us (280 workgroups), n = 512 72.8 / 80.1, n = 128 36.5 / 38.8 (112),
+// 5760x2880 n = 256 27.5 / 32.0 (92), n = 512 37.9 / 41.8; but 14336x4096 n = 64 34.4 / 24.7 (56), 4096x14336 n = 512 111 /
+// 84 (128). A whole k of 64-row waves split like the others measures as the 32-row waves do.
+static int mx4_rt(int m, int k, int ncb) {
+    return m >= 512 && (m + 255) / 256 * ncb >= (k <= 4096 ? 88 : 256) ? 2 : 1;
+}
+static hipError_t mx4_go(const WeightView& w, const GemmAct& A, int m, int n, float* c, int ldc, hipStream_t st, float* part,
+                         const Epi& ep) {
+    const int ncb = A.NP / 64, rt = mx4_rt(m, A.K, ncb), total = (m + 128 * rt - 1) / (128 * rt) * ncb;
+    int ns = 1, sb_per = 0;
+    if (rt == 1 && part != nullptr) split_plan(total, A.Kp / 256, &ns, &sb_per);
+    if (ns == 1) return launch_mx4_gemm(w, A, m, n, c, ldc, st, Groups{}, rt, 1, 0, tail_split(total), 0, ep);
+    const int64_t slice = (int64_t) n * m;
+    const hipError_t e = launch_mx4_gemm(w, A, m, n, part, m, st, Groups{}, rt, ns, sb_per, 0, slice, Epi{});
+    return e != hipSuccess ? e : launch_split_reduce(part, ns, slice, m, n, c, ldc, st, ep);
+}
+
 size_t gemm_mma_split_floats(int dt, int k, int m, int n) {
     if (dt != Q4_K && dt != Q5_K && dt != Q6_K && dt != MXFP4 && dt != Q4_0 && dt != Q8_0 && dt != NVFP4 && dt != Q1_0)
         return 0;
@@ -1064,7 +987,7 @@ hipError_t launch_gemm_mma(int dt, const WeightView& w, const GemmAct& A, int k,
     case Q4_0: return kq_go<Q4_0, 1, 2>(w, A, m, n, c, ldc, st, Groups{}, part, ep);
     case Q8_0: return kq_go<Q8_0, 1, 2>(w, A, m, n, c, ldc, st, Groups{}, part, ep);
     case Q6_K: return kq_go<Q6_K, 1, 2>(w, A, m, n, c, ldc, st, Groups{}, part, ep);
-    case MXFP4: return kq_go<MXFP4, 1, 2>(w, A, m, n, c, ldc, st, Groups{}, part, ep);
+    case MXFP4: return mx4_go(w, A, m, n, c, ldc, st, part, ep);
     default: return hipErrorNotSupported;
     }
 }
@@ -1079,7 +1002,8 @@ hipError_t launch_gemm_mma_grouped(int dt, const WeightView& w, const GemmAct& A
     case Q4_0: return kq_go<Q4_0, 1, 2>(w, A, g.gm, A.NP, c, ldc, st, g);
     case Q8_0: return kq_go<Q8_0, 1, 2>(w, A, g.gm, A.NP, c, ldc, st, g);
     case Q6_K: return kq_go<Q6_K, 1, 2>(w, A, g.gm, A.NP, c, ldc, st, g);
-    case MXFP4: return kq_go<MXFP4, 1, 2>(w, A, g.gm, A.NP, c, ldc, st, g);
+    case MXFP4:   // cap64 slot blocks at the most: the real count is on the device
+        return launch_mx4_gemm(w, A, g.gm, A.NP, c, ldc, st, g, mx4_rt(g.gm, A.K, cap64), 1, 0, 0, 0, Epi{});
     default: return hipErrorNotSupported;
     }
 }

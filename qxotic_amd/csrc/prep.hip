@@ -46,18 +46,19 @@ __global__ void __launch_bounds__(256) quant_f2_kernel(const float* __restrict__
 // chunk store of 32 threads fills 512 contiguous bytes; a group past the row's last block, and every row
 // past `rows` in the last tile, is zero-filled. Runs once per pinned tensor.
 //
-// Q8_0, Q4_0 and MXFP4 groups are also checked for the matrix-core GEMM (mma.hip), which folds each block's
-// scale into an f16 weight operand relative to a per-row, per-group reference: MXFP4 codes times
-// 2^(e_b - e_ref + 1), Q4_0 / Q8_0 codes times d_b·2^s_r with s_r set by the group's largest fp16 exponent.
-// That is exact while every folded operand is a normal f16 (>= 2^-14). A block whose products are zero
-// whatever its scale (MXFP4: every code 0 or -0; Q8_0: every q 0) must not set the reference, or a large
-// scale on it would push its neighbours below f16's range: such a block's scale is stored as 0 (MXFP4 e=0,
+// Q8_0, Q4_0 and MXFP4 groups are also checked for the matrix-core GEMMs. mma.hip folds each Q4_0 / Q8_0 block's scale
+// into an f16 weight operand relative to a per-row, per-group reference: codes times d_b·2^s_r with s_r set by the
+// group's largest fp16 exponent. That is exact while every folded operand is a normal f16 (>= 2^-14). A block whose
+// products are zero whatever its scale (MXFP4: every code 0 or -0; Q8_0: every q 0) must not set the reference, or a
+// large scale on it would push its neighbours below f16's range: such a block's scale is stored as 0 (MXFP4 e=0,
 // Q8_0 d=0; its terms are zero on every path either way) and the reference comes from the other blocks. A
 // Q4_0 block always counts (jam's n >= 8 term -fl(8d)·fl(xs0+xs1) does not vanish with the codes). A group
-// whose blocks still span more than the f16 range below its reference (MXFP4 e_b < e_ref - 14; Q8_0
-// |d_b| < 2^(F - 36), Q4_0 |d_b| < 2^(F - 39), F the largest fp16 exponent field), or that holds a non-finite
+// whose blocks still span more than the f16 range below its reference (Q8_0 |d_b| < 2^(F - 36), Q4_0
+// |d_b| < 2^(F - 39), F the largest fp16 exponent field), or that holds a non-finite
 // scale (MXFP4 e = 255, which jam decodes as +Inf; an fp16 Inf/NaN), sets *flag: the host then keeps the
-// tensor off the matrix cores, on kernels that apply every block scale in f32 as jam does.
+// tensor off the matrix cores, on kernels that apply every block scale in f32 as jam does. MXFP4's kernel (mx4.hip) needs
+// e <= MX4_MAX_E alone; tensors with blocks 15 or more binades below their group's largest stay on the other kernels
+// too, which take them as before.
 template <int DT>
 __global__ void __launch_bounds__(256) repack_kernel(const uint8_t* __restrict__ raw, int64_t raw_stride,
                                                      int64_t rows, int64_t rb, int64_t G, uint8_t* __restrict__ qs,
@@ -141,19 +142,16 @@ __global__ void __launch_bounds__(256) repack_kernel(const uint8_t* __restrict__
             }
         }
         bool bad = false;   // the matrix cores' folding would not be exact for this row's group
-        if constexpr (DT == MXFP4) {   // byte 8: the reference exponent (largest of the counted blocks); 9..11
-                                       // zero; 12..15: the f32 2^(e_ref - 128) that the matrix cores apply per group
+        if constexpr (DT == MXFP4) {   // byte 8: the largest exponent of the counted blocks; 9..15 zero
             uint8_t er = 0;
             for (int j = 0; j < BPG; j++) {
                 if (!nz[j] && ds[j] != 255) ds[j] = 0;
                 er = ds[j] > er ? ds[j] : er;
                 bad |= ds[j] == 255;
             }
-            for (int j = 0; j < BPG; j++) bad |= nz[j] && (int) ds[j] + 14 < (int) er;
+            for (int j = 0; j < BPG; j++) bad |= nz[j] && ((int) ds[j] + 14 < (int) er || ds[j] > MX4_MAX_E);
             ds[8] = er;
-            for (int t = 9; t < 12; t++) ds[t] = 0;
-            const uint32_t f = __builtin_bit_cast(uint32_t, e8m0_half(er));
-            for (int t = 0; t < 4; t++) ds[12 + t] = (uint8_t) (f >> (8 * t));
+            for (int t = 9; t < 16; t++) ds[t] = 0;
         } else {
             uint32_t hs[BPG];
             int F = 0;   // largest fp16 exponent field of the group
@@ -224,11 +222,10 @@ constexpr int PREP_GRID = 1024;      // a multiple of 8 (XCDs)
 // with NaN/overflow -> -128, and the per-16 sums in _mm512_reduce_add_ps's pairing (distance 8, 4, 2, 1),
 // all inside the lane. A lane holds elements 16h..16h+15 of its block (half h), or for MXO elements
 // 8h..8h+7 and 16+8h..16+8h+7: exactly the two (K-step, half) planes it stores.
-// MXO: the MXFP4 element order (the GEMM converts a weight byte's two nibbles, elements e and e + 16 of the
-// block, into one f16 pair): K-step 2·block + ks, half q, slot i holds element 8q + 4ks + i/2 + 16·(i % 2).
+// MXO: the MXFP4 element order (a weight byte's two nibbles are elements e and e + 16 of the block).
 // ORD: the element order of the codes inside a K-step, matching the weight operand the GEMM builds:
 //   0  elements 16q + 8ks + perm8(i)            (nibble / byte fields, Q4_K, Q5_K, Q6_K, Q4_0, Q8_0, Q1_0)
-//   1  pairs (e, e + 16) of the 32-block         (MXFP4: a weight byte's two e2m1 codes)
+//   1  pairs (e, e + 16) of the 32-block, as two 6-bit digits per code (MXFP4; GemmAct::b8)
 //   2  pairs (u, u + 8) of each 16-element sub-block, K-step ks = sub-block ks of the block (NVFP4)
 // f1all: jam's F1 quantization for every slot (NVFP4, whose only jam path is F1 at every n, jam.c:662-668).
 template <int SK, int ORD, int SG>
@@ -352,14 +349,36 @@ __global__ void __launch_bounds__(256) gemm_prep(const float* __restrict__ a, in
                             qf[i] = ok ? fminf(fmaxf(rintf(p), -128.0f), 127.0f) : -128.0f;
                         }
                     }
+                    if constexpr (ORD == 1) {
+                        // sign and two digits per code, |q| = 16·h + l, 6 bits each (fp6 e2m3: sign, then the digit);
+                        // position 2j + p of the half is element j + 16p (qf[j + 8p]), as in a weight's nibbles
+                        uint32_t h[3] = {0, 0, 0}, l[3] = {0, 0, 0};
+#pragma unroll
+                        for (int i = 0; i < 16; i++) {
+                            const int v = (int) qf[(i >> 1) + 8 * (i & 1)], av = v < 0 ? -v : v, sg = v < 0 ? 32 : 0;
+                            const uint32_t hd = (uint32_t) ((av >> 4) | sg), ld = (uint32_t) ((av & 15) | sg);
+                            const int w = 6 * i / 32, o = 6 * i % 32;
+                            h[w] |= hd << o, l[w] |= ld << o;
+                            if (o > 26) h[w + 1] |= hd >> (32 - o), l[w + 1] |= ld >> (32 - o);
+                        }
+                        // the halves trade: half 0 stores the block's high digits, half 1 its low digits
+                        uint32_t o[3];
+#pragma unroll
+                        for (int i = 0; i < 3; i++)
+                            o[i] = __builtin_bit_cast(uint32_t, pair_other<SG>(__builtin_bit_cast(float, hh ? h[i] : l[i])));
+                        const int64_t at = (int64_t) (2 * b + hh) * NP + t;
+                        uint8_t* p16 = reinterpret_cast<uint8_t*>(bq);
+                        uint8_t* p8 = p16 + (int64_t) Kp * NP;
+                        *reinterpret_cast<uint4*>(p16 + at * 16) = hh ? make_uint4(o[0], o[1], o[2], l[0]) : make_uint4(h[0], h[1], h[2], o[0]);
+                        *reinterpret_cast<uint2*>(p8 + at * 8) = hh ? make_uint2(l[1], l[2]) : make_uint2(o[1], o[2]);
+                    }
                     // the thread's two (K-step, half) planes: 8 f16 (16 bytes) each at the slot
 #pragma unroll
-                    for (int ks = 0; ks < 2; ks++) {
+                    for (int ks = 0; ks < (ORD == 1 ? 0 : 2); ks++) {
                         half8 hv;
 #pragma unroll
                         for (int i = 0; i < 8; i++) {
                             if constexpr (ORD == 0) hv[perm8(i)] = (_Float16) qf[8 * ks + i];   // elements 16hh + 8ks + i
-                            else if constexpr (ORD == 1) hv[2 * (i & 3) + (i >> 2)] = (_Float16) qf[8 * (i >> 2) + 4 * ks + (i & 3)];
                             // ORD 2: slot 2j = element 16ks + 4hh + j, slot 2j + 1 = element 16ks + 4hh + 8 + j
                             else hv[2 * (i & 3) + (i >> 2)] = (_Float16) qf[8 * ks + 4 * (i >> 2) + (i & 3)];
                         }
@@ -420,7 +439,8 @@ __global__ void __launch_bounds__(256) gemm_prep(const float* __restrict__ a, in
             // consecutive entries of a slot's 8 / 16 sums (shi, slo)
             for (int i = threadIdx.x; i < nbp * SG; i += 256) {
                 const int sl = i % SG, b = i / SG;
-                dx[(int64_t) b * NP + t0 + sl] = lsm[sl * 3 * nbp + b] * ldexpf(1.0f, -slot_exp(sl));
+                const int64_t at = ORD == 1 ? ((int64_t) (b >> 2) * NP + t0 + sl) * 4 + (b & 3) : (int64_t) b * NP + t0 + sl;
+                dx[at] = lsm[sl * 3 * nbp + b] * ldexpf(1.0f, -slot_exp(sl));
             }
             if constexpr (SK != 0) {
                 constexpr int NS = SK == 1 ? 8 : 16;   // sums per slot and group of 8 blocks
@@ -464,7 +484,7 @@ static hipError_t prep_np(int dt, const float* a, int lda, int n, int NP, int k,
     _Float16* slo = (_Float16*) (p + sb);
     p += 2 * sb;
     float* es = (float*) p;
-    *out = GemmAct{bq, dx, shi, slo, es, NP, Kp, k};
+    *out = GemmAct{bq, dx, shi, slo, es, (const uint8_t*) bq + (int64_t) Kp * NP, NP, Kp, k};
     if (NP <= 0) return hipSuccess;
     const int vec = ((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (lda & 3) == 0) ? 1 : 0;
     const int kind = dt == MXFP4 ? 3 : dt == NVFP4 ? 4 : sk;
