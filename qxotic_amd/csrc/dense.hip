@@ -7,7 +7,7 @@
 // and f32 x f32 products are formed exactly by the FMA / the matrix cores); only the f32 summation order
 // differs from jam's.
 //
-// Layout. A device copy keeps the rows row-major, each padded with zeros to a 256-byte pitch (WeightView::G),
+// Layout. A device copy keeps the rows row-major, each padded with zeros to a pitch of an odd multiple of 256 bytes (WeightView::G),
 // so every row starts 16-byte aligned and a 16-byte load never crosses into the next row.
 //
 // Kernels.
@@ -19,6 +19,8 @@
 //  * dense_mma_kernel (F16, and BF16 with rounded activations, past the GEMV): LDS-staged f16 / bf16 matrix cores.
 #include "common.h"
 #include "launch.h"
+
+#include <type_traits>
 
 namespace jamhip {
 
@@ -346,7 +348,7 @@ __global__ void __launch_bounds__(64 * DT_WAVES) dense_tile_kernel(WeightView w,
 // F16 weights and BF16 weights with bf16-rounded activations (k even or k % 32 == 0: jam's bf16 kernels) run
 // on the f16 / bf16 matrix cores with LDS-staged operands, the structure of the quantized prefill GEMM
 // (mma.hip) without its per-block scales:
-//  * dense_prep_kernel (one workgroup per token) writes the activations in the MFMA operand order, planes
+//  * dense_prep_kernel writes the activations in the MFMA operand order, planes
 //    [Kp/16 K-steps][2 halves][NP slots][8] (half h = elements 8h..8h+7 of the K-step, zero past k): for F16
 //    weights the f16 high part and f16 remainder of x·2^-e_t, e_t putting the token's largest |x| in
 //    [2^14, 2^15) (hi + lo hold x to about 22 bits), and es[t] = 2^e_t; for BF16 weights jam's bf16(x), es = 1.
@@ -370,40 +372,60 @@ size_t dense_act_bytes(int dt, int n, int k) {
     return pl * plane + ((size_t) dense_np(n) * 4 + 255) / 256 * 256;
 }
 
-__global__ void __launch_bounds__(256) dense_prep_kernel(const float* __restrict__ a, int lda, int n, int k, int Kp,
+// A workgroup of 8 waves takes 8 tokens and one of gridDim.y runs of their rows: each wave first finds its token's largest
+// |x| (the whole row, from L2 past the first workgroup), then 8 consecutive threads store one 8-element row of the
+// operand for the 8 tokens, a whole 128-byte line. One workgroup per token stored 16 bytes of each line and read its
+// row alone: 512 x 4096 15.6 -> 9.2 us.
+__global__ void __launch_bounds__(512) dense_prep_kernel(const float* __restrict__ a, int lda, int n, int k, int Kp,
                                                          int NP, int hl, uint16_t* __restrict__ hi,
                                                          uint16_t* __restrict__ lo, float* __restrict__ es) {
-    __shared__ float wmax[4];
-    const int t = blockIdx.x;
-    const float* x = a + (int64_t) t * lda;
-    float down = 1.0f;
-    if (hl) {   // the token's largest |x|; a non-finite one leaves the scale at 1 (the outputs go non-finite)
+    __shared__ float sdown[8];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int t0 = 8 * blockIdx.x;
+    if (hl && t0 + wave < n) {   // a non-finite largest |x| leaves the scale at 1 (the outputs go non-finite)
+        const float* x = a + (int64_t) (t0 + wave) * lda;
         float mx = 0.0f;
-        for (int e = threadIdx.x; e < k; e += 256) mx = fmaxf(mx, fabsf(x[e]));
+        if ((reinterpret_cast<uintptr_t>(x) & 15) == 0) {
+            const int k4 = k / 4;
+#pragma unroll 8
+            for (int e = lane; e < k4; e += 64) {
+                const float4 f = reinterpret_cast<const float4*>(x)[e];
+                mx = fmaxf(fmaxf(mx, fmaxf(fabsf(f.x), fabsf(f.y))), fmaxf(fabsf(f.z), fabsf(f.w)));
+            }
+            for (int e = 4 * k4 + lane; e < k; e += 64) mx = fmaxf(mx, fabsf(x[e]));
+        } else {
+#pragma unroll 8
+            for (int e = lane; e < k; e += 64) mx = fmaxf(mx, fabsf(x[e]));
+        }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-        if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
-        __syncthreads();
-        mx = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-        int ex;
+        int ex = 0;
         if (mx > 0.0f && mx <= 3.40282347e38f) {
             int e2;
             frexpf(mx, &e2);   // mx in [2^(e2-1), 2^e2)
             ex = 15 - e2;
             ex = ex > 126 ? 126 : ex;
-        } else {
-            ex = 0;
         }
-        down = ldexpf(1.0f, ex);
-        if (threadIdx.x == 0) es[t] = ldexpf(1.0f, -ex);
-    } else if (threadIdx.x == 0) {
-        es[t] = 1.0f;
+        if (lane == 0) {
+            sdown[wave] = ldexpf(1.0f, ex);
+            if (blockIdx.y == 0) es[t0 + wave] = ldexpf(1.0f, -ex);
+        }
+    } else if (!hl && blockIdx.y == 0 && lane == 0 && t0 + wave < n) {
+        es[t0 + wave] = 1.0f;
     }
+    __syncthreads();
+    const int t = t0 + (threadIdx.x & 7);
+    if (t >= n) return;   // after the only barrier
+    const float* x = a + (int64_t) t * lda;
+    const float down = hl ? sdown[threadIdx.x & 7] : 1.0f;
+    const bool vec = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
     // 8-element runs: run g = elements 8g..8g+7 = K-step g / 2, half g % 2
-    for (int g = threadIdx.x; g < Kp / 8; g += 256) {
+    const int ng = Kp / 8, per = (ng + (int) gridDim.y - 1) / (int) gridDim.y;
+    const int g1 = min(ng, per * ((int) blockIdx.y + 1));
+    for (int g = per * (int) blockIdx.y + (threadIdx.x >> 3); g < g1; g += 64) {
         float v[8];
         const int e0 = 8 * g;
-        if (e0 + 8 <= k && ((reinterpret_cast<uintptr_t>(x + e0) & 15) == 0)) {
+        if (vec && e0 + 8 <= k) {
             const float4 f0 = *reinterpret_cast<const float4*>(x + e0), f1 = *reinterpret_cast<const float4*>(x + e0 + 4);
             v[0] = f0.x, v[1] = f0.y, v[2] = f0.z, v[3] = f0.w, v[4] = f1.x, v[5] = f1.y, v[6] = f1.z, v[7] = f1.w;
         } else {
@@ -429,6 +451,7 @@ __global__ void __launch_bounds__(256) dense_prep_kernel(const float* __restrict
 
 typedef _Float16 half8d __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) void lds_void_d;
+typedef uint32_t u32x4d __attribute__((ext_vector_type(4)));
 
 template <bool HL>
 __global__ void __launch_bounds__(256, 2) dense_mma_kernel(WeightView w, const uint16_t* __restrict__ xh,
@@ -526,6 +549,165 @@ __global__ void __launch_bounds__(256, 2) dense_mma_kernel(WeightView w, const u
     }
 }
 
+// Calls with many tokens: the same operands in tiles of 256 rows x 128 tokens, 8 waves of 64 x 64 (4 x 2), k in stages of
+// 64. The 128 x 64 kernel above moves 512 bytes (F16) global -> LDS per 128 x 64 outputs and k, and its waves wait for
+// those copies (26% MFMA busy); here it is 1024 bytes per 256 x 128, each fragment read from LDS feeds two MFMAs per
+// plane, and a stage's copies run during the whole stage before it (two LDS buffers, one workgroup per CU). A stage is 1536
+// cycles of LDS reads and 2048 of products on each SIMD (F16): its two waves take turns, one reading while the other
+// multiplies. With the prep, 128 x 64 kernel -> this one: F16 14336x4096 n = 512 243 -> 126 us, n = 2048 825 -> 486, BF16 n = 512
+// 197 -> 96; it then moves about 8 TB/s global -> LDS. Four buffers of 32 measured slower (140 us: the compiler makes LDS
+// reads wait for copies in flight to the other buffers).
+// LDS: weights [256 rows][128 B], the row's 16-byte piece p at position p ^ (row % 8), so that a fragment read's 8 lanes
+// per cycle fall on different banks (the copy writes lane-linear: the lane picks its source piece instead); activations
+// as prepared, [PL][8 8-element rows][128 tokens][16 B].
+
+template <bool HL>
+__global__ void __launch_bounds__(512, 1) dense_big_kernel(WeightView w, const uint16_t* __restrict__ xh,
+                                                           const uint16_t* __restrict__ xl, const float* __restrict__ es,
+                                                           int NP, int Kp, int k, int m, int n, float* __restrict__ c,
+                                                           int ldc, int nrb, int ncb, int st_per, int64_t c_slice,
+                                                           Epi ep) {
+    constexpr int PL = HL ? 2 : 1, A_BYTES = 256 * 128, BYTES = A_BYTES + PL * 16384;
+    __shared__ __align__(1024) unsigned char sb0[BYTES], sb1[BYTES];
+    const int total = nrb * ncb, lin = tile_of_block(false, total);
+    if (lin >= total) return;
+    const int rb = lin / ncb, cb = lin % ncb;
+    const int lane = threadIdx.x & 63, r = lane & 31, q = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = wave >> 1, wt = wave & 1;
+    const int64_t row0 = (int64_t) rb * 256;
+    const int n0 = cb * 128;
+    const int nstk = Kp / DMM_STAGE;
+    const int st0 = st_per > 0 ? st_per * (int) blockIdx.y : 0;
+    const int nst = st_per > 0 ? min(nstk, st0 + st_per) : nstk;
+    // weights: the wave copies rows 32·wave.. in four pieces of 8 rows x 128 bytes
+    const uint8_t* asrc[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int lr = 32 * wave + 8 * i + (lane >> 3);
+        const int64_t row = row0 + lr < m ? row0 + lr : m - 1;
+        asrc[i] = w.qs + (w.r0 + row) * w.G + 16 * ((lane & 7) ^ (lr & 7));
+    }
+    // activations: 8-element row `wave` of the stage, tokens 0..63 and 64..127; a last half block re-reads its first slots
+    const int t1 = n0 + 64 < NP ? 64 : 0;
+    const uint16_t* bsrc = xh + ((int64_t) wave * NP + n0) * 8 + 8 * lane;
+    const int64_t plane_off = xl - xh;
+    auto issue = [&](int st, unsigned char* buf) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            __builtin_amdgcn_global_load_lds(asrc[i] + (int64_t) st * (DMM_STAGE * 2),
+                                             (lds_void_d*) (buf + wave * 4096 + i * 1024), 16, 0, 0);
+#pragma unroll
+        for (int pl = 0; pl < PL; pl++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                __builtin_amdgcn_global_load_lds(bsrc + pl * plane_off + ((int64_t) (8 * st) * NP + h * t1) * 8,
+                                                 (lds_void_d*) (buf + A_BYTES + pl * 16384 + wave * 2048 + h * 1024), 16, 0,
+                                                 0);
+    };
+    floatx16 acc[2][2] = {{floatx16{}, floatx16{}}, {floatx16{}, floatx16{}}};
+    u32x4d af[4][2], bf[4][PL][2];   // a stage's fragments [K-step][..]
+    auto read = [&](auto U, int st) __attribute__((always_inline)) {
+        const unsigned char* buf = decltype(U)::value ? sb1 : sb0;
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int lr = 64 * wr + 32 * i + r;
+                af[ks][i] = *reinterpret_cast<const u32x4d*>(buf + lr * 128 + (((2 * ks + q) ^ (lr & 7)) * 16));
+            }
+#pragma unroll
+            for (int pl = 0; pl < PL; pl++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    bf[ks][pl][j] = *reinterpret_cast<const u32x4d*>(buf + A_BYTES + pl * 16384 + (2 * ks + q) * 2048 +
+                                                                    (64 * wt + 32 * j + r) * 16);
+        }
+        if (DMM_STAGE * (st + 1) > k) {   // the stage holding column k - 1: columns >= k -> 0 (they may hold anything)
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const int e0 = DMM_STAGE * st + 16 * ks + 8 * q;
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        if (e0 + e >= k) af[ks][i][e >> 1] &= (e & 1) ? 0x0000ffffu : 0xffff0000u;
+                }
+        }
+        __builtin_amdgcn_sched_barrier(0);   // the phases stay apart: reads | copies | products
+    };
+    auto mul = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+            for (int pl = 0; pl < PL; pl++)
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        if constexpr (HL)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8d, af[ks][i]),
+                                                                               __builtin_bit_cast(half8d, bf[ks][pl][j]), acc[i][j], 0, 0, 0);
+                        else
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[ks][i]),
+                                                                                __builtin_bit_cast(bf16x8, bf[ks][pl][j]), acc[i][j], 0, 0, 0);
+                    }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto copies_in = [&]() { __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8)); };   // vmcnt(0): this wave's copies
+    auto meet = [&]() {
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    constexpr std::integral_constant<int, 0> b0{};
+    constexpr std::integral_constant<int, 1> b1{};
+    // Waves 0..3 (one per SIMD) read stage s in half-step 2s and multiply in 2s + 1; waves 4..7 a half-step later. Buffer
+    // s % 2 is last read in 2s + 1, refilled with stage s + 2 from 2s + 2 on (each wave its own pieces) and complete, by
+    // every wave's wait before the barrier that ends it, with 2s + 3.
+    issue(st0, sb0);
+    copies_in();
+    meet();
+    if (wave < 4) {
+        auto step = [&](auto U, int st) __attribute__((always_inline)) {
+            read(U, st);
+            if (st + 1 < nst) issue(st + 1, decltype(U)::value ? sb0 : sb1);
+            meet();
+            mul();
+            copies_in();
+            meet();
+        };
+        for (int st = st0; st < nst; st += 2) {
+            step(b0, st);
+            if (st + 1 < nst) step(b1, st + 1);
+        }
+        meet();   // the other waves' last half-step
+    } else {
+        if (st0 + 1 < nst) issue(st0 + 1, sb1);
+        meet();
+        auto step = [&](auto U, int st) __attribute__((always_inline)) {
+            read(U, st);
+            copies_in();
+            meet();
+            if (st + 2 < nst) issue(st + 2, decltype(U)::value ? sb1 : sb0);
+            mul();
+            meet();
+        };
+        for (int st = st0; st < nst; st += 2) {
+            step(b0, st);
+            if (st + 1 < nst) step(b1, st + 1);
+        }
+    }
+    if (st_per > 0) c += (int64_t) blockIdx.y * c_slice;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int t = n0 + 64 * wt + 32 * j + r;
+        if (t >= n) continue;
+        const float sc = es[t];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            store_column(c + (int64_t) t * ldc, row0 + 64 * wr + 32 * i + 4 * q, m, acc[i][j], sc, ep, st_per > 0);
+    }
+}
+
 // ----------------------------------------------------------------------------------------- launchers
 // jam rounds BF16's activations to bf16 where its bf16 kernels take the call (jam.c:622-652).
 static bool bf16_rounds(int n, int k) { return (n >= 8 && k % 2 == 0) || k % 32 == 0; }
@@ -613,6 +795,10 @@ static void dense_split(int total, int nstk, int* ns, int* st_per) {
     *ns = want > 1 ? (nstk + *st_per - 1) / *st_per : 1;
 }
 
+// Workgroups (K slices included) from which dense_big_kernel, one per CU, beats the 128 x 64 one: 128 of them: F16 4096x14336
+// n = 512 190 against 252 us, 4096x4096 n = 256 44.5 / 51; 56 x 5 (14336x4096 n = 128) 64 / 99.
+constexpr int DBG_MIN_TILES = 128;
+
 size_t dense_mma_split_floats(int dt, int k, int m, int n) {
     if (!dense_mma_planes(dt, n, k)) return 0;
     int ns, st_per;
@@ -629,22 +815,31 @@ hipError_t launch_dense_mma(int dt, const WeightView& w, const float* a, int lda
     uint16_t* xh = (uint16_t*) scratch;
     uint16_t* xl = (uint16_t*) ((uint8_t*) scratch + plane);
     float* es = (float*) ((uint8_t*) scratch + pl * plane);
-    dense_prep_kernel<<<n, 256, 0, st>>>(a, lda, n, k, Kp, NP, pl == 2, xh, pl == 2 ? xl : xh, es);
-    const int nrb = (m + 127) / 128, ncb = NP / 64, total = nrb * ncb;
-    int ns, st_per;
-    dense_split(total, Kp / DMM_STAGE, &ns, &st_per);
+    // about two workgroups per CU, each with at least one pass of 64 runs
+    const int ptiles = (n + 7) / 8, pmax = (Kp / 8 + 63) / 64, pwant = (512 + ptiles - 1) / ptiles;
+    dense_prep_kernel<<<dim3((unsigned) ptiles, (unsigned) (pwant < pmax ? pwant : pmax)), 512, 0, st>>>(a, lda, n, k, Kp, NP, pl == 2, xh, pl == 2 ? xl : xh, es);
+    int nrb = (m + 127) / 128, ncb = NP / 64, ns, st_per;
+    dense_split(nrb * ncb, Kp / DMM_STAGE, &ns, &st_per);
     if (ns > 1 && part == nullptr) return hipErrorInvalidValue;
-    const int grid = tile_grid(false, total);
     float* out = ns > 1 ? part : c;
     const int ldo = ns > 1 ? m : ldc;
     const int64_t slice = (int64_t) n * m;
-    const size_t lds = 2 * (size_t) (4 * 4096 + pl * 8192);
-    if (pl == 2)
-        dense_mma_kernel<true><<<dim3(grid, ns), 256, lds, st>>>(w, xh, xl, es, NP, Kp, k, m, n, out, ldo, nrb, ncb,
-                                                                 st_per, slice, ns > 1 ? Epi{} : ep);
-    else
-        dense_mma_kernel<false><<<dim3(grid, ns), 256, lds, st>>>(w, xh, xh, es, NP, Kp, k, m, n, out, ldo, nrb, ncb,
-                                                                  st_per, slice, ns > 1 ? Epi{} : ep);
+    const Epi epo = ns > 1 ? Epi{} : ep;
+    const int brb = (m + 255) / 256, bcb = (NP + 127) / 128;
+    if (brb * bcb * ns >= DBG_MIN_TILES) {   // the same K slices
+        const dim3 grid((unsigned) tile_grid(false, brb * bcb), (unsigned) ns);
+        if (pl == 2)
+            dense_big_kernel<true><<<grid, 512, 0, st>>>(w, xh, xl, es, NP, Kp, k, m, n, out, ldo, brb, bcb, st_per, slice, epo);
+        else
+            dense_big_kernel<false><<<grid, 512, 0, st>>>(w, xh, xh, es, NP, Kp, k, m, n, out, ldo, brb, bcb, st_per, slice, epo);
+    } else {
+        const dim3 grid((unsigned) tile_grid(false, nrb * ncb), (unsigned) ns);
+        const size_t lds = 2 * (size_t) (4 * 4096 + pl * 8192);
+        if (pl == 2)
+            dense_mma_kernel<true><<<grid, 256, lds, st>>>(w, xh, xl, es, NP, Kp, k, m, n, out, ldo, nrb, ncb, st_per, slice, epo);
+        else
+            dense_mma_kernel<false><<<grid, 256, lds, st>>>(w, xh, xh, es, NP, Kp, k, m, n, out, ldo, nrb, ncb, st_per, slice, epo);
+    }
     if (ns > 1) return launch_split_reduce(part, ns, slice, m, n, c, ldc, st, ep);
     return hipGetLastError();
 }

@@ -51,3 +51,31 @@ def test_short_dense(hip, dt, m, n, k):
             assert (np.abs(fused - whole) <= bound + 2.0 ** -23 * (np.abs(ref) + np.abs(bias) + np.abs(c0))).all()
     finally:
         hip.evict(Segment.of(w))
+
+
+# n past 64 with enough tiles: 256 x 128 workgroups, 64 of k per stage; whole, split and masked last stages, ragged edges
+@pytest.mark.parametrize("m,n,k", [(4096, 1024, 64), (3870, 1000, 100), (257, 129, 8200), (8192, 513, 36), (2048, 65, 4100), (4224, 512, 330)])
+@pytest.mark.parametrize("dt", [O.F16, O.BF16])
+def test_dense_wide_tiles(hip, dt, m, n, k):
+    """F16 products are exact in f32, x kept to 22 bits; any order of k sums errs by at most (k + 2)·2^-24·sum|w*a| and the
+    dropped remainder of x by 2^-22 of it. BF16 activations are rounded first, products exact."""
+    import torch
+    from qxotic_amd.jam import JAM, Segment
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    w = (torch.randn((m, k + 24), generator=g, device="cuda") * 0.02).to(torch.float16 if dt == O.F16 else torch.bfloat16)
+    w[:, k:] = float("nan")   # the pinned rows go on past k
+    host = w.view(torch.uint8).cpu().numpy()
+    a = torch.randn((n, k), generator=g, device="cuda")
+    c = torch.full((n, m + 1), -7.0, device="cuda")
+    torch.cuda.synchronize()
+    assert hip.pin(Segment.of(host), dt, k + 24, m) == JAM.OK, hip.last_error()
+    try:
+        assert hip.mm_device(Segment.of(host), dt, k + 24, a.data_ptr(), k, c.data_ptr(), m + 1, m, n, k) == JAM.OK
+        hip.synchronize()
+        x = a.double() if dt == O.F16 else a.bfloat16().double()
+        w64 = w[:, :k].double()
+        bound = ((k + 2) * 2.0 ** -24 + 2.0 ** -22) * (x.abs() @ w64.abs().T)
+        assert ((c[:, :m].double() - x @ w64.T).abs() <= bound).all()
+        assert (c[:, m:] == -7.0).all()
+    finally:
+        hip.evict(Segment.of(host))
