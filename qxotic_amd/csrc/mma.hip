@@ -49,6 +49,9 @@ JAMHIP_DEV void dma16(const void* g, void* lds_base) {
     __builtin_amdgcn_global_load_lds(g, (lds_void*) lds_base, 16, 0, 0);
 }
 
+typedef __attribute__((address_space(3))) unsigned char lds_u8;
+JAMHIP_DEV void dma16l(const void* g, lds_u8* lds_base) { __builtin_amdgcn_global_load_lds(g, (lds_void*) lds_base, 16, 0, 0); }
+
 JAMHIP_DEV uint32_t hbits(_Float16 h) { return (uint32_t) __builtin_bit_cast(uint16_t, h); }
 JAMHIP_DEV uint32_t pack2(_Float16 lo, _Float16 hi) { return hbits(lo) | (hbits(hi) << 16); }
 
@@ -866,6 +869,289 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) kq_gemm_kernel(WeightView w, G
     }
 }
 
+// ------------------------------------------------------------------------------------------ wide kernel
+// The K-quants with more than 64 tokens: the same arithmetic, in waves of 32 rows x 128 tokens (a workgroup of 4 waves: 128
+// rows x 128 tokens), k in stages of 64 (two blocks). kq_gemm_kernel is bound by VALU issue (18 instructions per MFMA, a
+// third of them the weight decode): here a decoded fragment serves four token tiles instead of two (11 per MFMA), a stage's
+// copies go out at its start into a buffer of their own, fragments are read a step ahead, and products are issued between
+// the previous step's FMAs. Figures at wide_plan. Three stage buffers instead of two (Q4_K) measured slower (n = 512 116 us):
+// it is the copies' own issue and LDS traffic that cost, not their latency.
+// Stage buffer: weight chunks [4 tiles][NCS][32 rows][16 B], row headers [4][32][HB], codes [2 blocks][2 K-steps][2 halves][128
+// tokens][16 B], block scales [2][128] f32; the buffer of a super-block's sums stage (the last for Q4_K / Q5_K, the first for
+// Q6_K) also holds their hi and lo planes [128 tokens][SW] f16.
+// Q6_K takes a half super-block's blocks in the order 0, 2, 1, 3: blocks j and j + 2 are the two nibbles of the same chunks.
+template <int DT> struct WStage {
+    static constexpr int NCS = DT == Q4_K ? 2 : DT == Q5_K ? 4 : 5;   // Q5_K: nibbles, qh; Q6_K: ql, qh, scales
+    static constexpr int HB = DT == Q6_K ? 2 : 16, SW = DT == Q6_K ? 16 : 8;
+    static constexpr int SQ = DT == Q6_K ? 0 : 3;                      // the stage that carries the sums
+    static constexpr int H = 4 * NCS * 512, B = H + (128 * HB + 1023) / 1024 * 1024, DX = B + 16384, S = DX + 1024,
+                         BYTES = S + 2 * 128 * SW * 2;
+};
+
+template <int I, int N, typename F> JAMHIP_DEV void unroll(const F& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        unroll<I + 1, N>(f);
+    }
+}
+
+template <int DT>
+__global__ void __launch_bounds__(MMA_THREADS, 2) kq_wide_kernel(WeightView w, GemmAct A, int m, int n,
+                                                                 float* __restrict__ c, int ldc, int nrb, int ncb,
+                                                                 int64_t tiles, int sb_per, int64_t c_slice, Epi ep) {
+    using S = WStage<DT>;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    constexpr int NCS = S::NCS, NC = group_chunks(DT);
+    __shared__ __align__(1024) unsigned char sb0[S::BYTES], sb1[S::BYTES];
+    const int total = nrb * ncb, lin = tile_of_block(false, total);
+    if (lin >= total) return;
+    const int rb = lin / ncb, cb = lin % ncb;
+    const int64_t T0 = (int64_t) rb * 4;
+    const int n0 = cb * 128;
+    const int lane = threadIdx.x & 63, r = lane & 31, q = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int G = (int) w.G, nsb = A.Kp / 256;
+    const int g0 = sb_per * (int) blockIdx.y, g1 = sb_per > 0 ? min(nsb, g0 + sb_per) : nsb;   // super-blocks
+    const int64_t r0t = w.r0 >> 5;
+    const bool narrow = n - n0 <= 64;   // the last token block may hold 64 slots (NP is a multiple of 64)
+
+    // ---- copies: the wave's own row tile, a quarter of the codes, and one of the small pieces. Each source is a uniform
+    // pointer and a 32-bit lane offset (64-bit lane addresses would not fit beside the accumulators).
+    const int64_t Tw = T0 + wave < tiles ? T0 + wave : tiles - 1;
+    const int hi64 = narrow ? 0 : 64;   // a narrow block's second half re-reads the first
+    const uint32_t l16 = 16 * lane, rx = narrow ? (16 * r) & 255 : 16 * r;
+    // Q6_K's d: 16 B = 8 rows per lane, four lanes per tile (clamped like Tw)
+    const uint32_t h6 = DT == Q6_K ? (uint32_t) ((T0 + ((lane >> 2) & 3) < tiles ? (lane >> 2) & 3 : tiles - 1 - T0) * G * 64 + 16 * (lane & 3)) : 0;
+    // uniform sources of super-block g, advanced with it
+    const uint32_t np16 = (uint32_t) A.NP * 16, np64 = np16 * 4, np4 = np16 / 4;
+    constexpr int SWB = S::SW * 2, HS = 32 * S::HB;
+    const uint8_t* pa = w.qs + ((r0t + Tw) * G + g0) * (NC * CHUNK_STRIDE);
+    const uint8_t* ph = w.sc + ((r0t + (DT == Q6_K ? T0 : Tw)) * G + g0) * HS;
+    const uint8_t* pb = reinterpret_cast<const uint8_t*>(A.b) + (int64_t) (8 * g0) * np64 + (int64_t) (2 * (wave & 1)) * np16 + n0 * 16;
+    const uint8_t* px = reinterpret_cast<const uint8_t*>(A.dx) + (int64_t) (8 * g0) * np4 + n0 * 4;
+    const uint8_t* ps = reinterpret_cast<const uint8_t*>(wave >= 2 ? A.slo : A.shi) + ((int64_t) g0 * A.NP + n0) * SWB;
+    auto issue = [&](auto QD, auto NEXT) __attribute__((always_inline)) {   // stage qd (of the next super-block) -> buffer qd % 2
+        constexpr int qd = decltype(QD)::value, nx = decltype(NEXT)::value;
+        lds_u8* buf = (lds_u8*) (qd & 1 ? sb1 : sb0);
+        const uint8_t* ag = pa + nx * NC * CHUNK_STRIDE;
+        lds_u8* la = buf + wave * NCS * 512;
+        // K position of the stage's block bl: 32-block 8g + kb(bl)
+        constexpr int kb0 = 8 * nx + (DT == Q6_K ? 4 * (qd >> 1) + (qd & 1) : 2 * qd), kb1 = DT == Q6_K ? kb0 + 2 : kb0 + 1;
+        if constexpr (DT == Q6_K) {   // ql chunks 2·qd, 2·qd + 1; qh chunks 8 + 2h, 9 + 2h; the scales chunk 12
+            dma16l(ag + 2 * qd * CHUNK_STRIDE + l16, la);
+            dma16l(ag + (8 + 2 * (qd >> 1)) * CHUNK_STRIDE + l16, la + 1024);
+            if (lane < 32) dma16l(ag + 12 * CHUNK_STRIDE + l16, la + 2048);
+            if (wave == 0 && lane < 16) dma16l(ph + nx * HS + h6, buf + S::H);
+        } else {
+            dma16l(ag + 2 * qd * CHUNK_STRIDE + l16, la);
+            if constexpr (DT == Q5_K) dma16l(ag + 8 * CHUNK_STRIDE + l16, la + 1024);
+            if (lane < 32) dma16l(ph + nx * HS + l16, buf + S::H + wave * 512);
+        }
+        // codes: plane rows (block wave / 2, K-step wave % 2), halves 0 and 1, 128 tokens each
+        const uint8_t* bp = pb + (wave >> 1 ? kb1 : kb0) * np64;
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+                dma16l(bp + h * np16 + t * hi64 * 16 + l16, buf + S::B + (wave * 2 + h) * 2048 + t * 1024);
+        if (wave == 3) dma16l(px + kb0 * np4 + (rx + q * (uint32_t) ((kb1 - kb0) * np4)), buf + S::DX);
+        if constexpr (qd == S::SQ) {   // sums: 1 KB pieces of the planes [128 tokens][SW], waves 0, 1 hi, 2, 3 lo
+            constexpr int PCS = 128 * SWB / 1024;   // 2 or 4 pieces per plane
+#pragma unroll
+            for (int i = 0; i < PCS / 2; i++) {
+                const int p = (wave & 1) * (PCS / 2) + i;
+                dma16l(ps + nx * (A.NP * SWB) + (narrow ? p % (PCS / 2) : p) * 1024 + l16,
+                       buf + S::S + (wave >> 1) * 128 * SWB + p * 1024);
+            }
+        }
+    };
+    auto advance = [&]() __attribute__((always_inline)) {
+        pa += NC * CHUNK_STRIDE, ph += HS, pb += 8 * (int64_t) np64, px += 8 * (int64_t) np4, ps += (int64_t) A.NP * SWB;
+    };
+
+    uint32_t vmask_lo, vmask_hi, vmask_qh;   // in VGPRs: the mask-and-or is then one instruction
+    asm volatile("v_mov_b32 %0, 0x000F000F" : "=v"(vmask_lo));
+    asm volatile("v_mov_b32 %0, 0x00F000F0" : "=v"(vmask_hi));
+    asm volatile("v_mov_b32 %0, 0x00300030" : "=v"(vmask_qh));
+    (void) vmask_qh;
+
+    floatx16 acc[4], accs[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) acc[j] = accs[j] = floatx16{};
+    // integer offsets from the buffer, so that the compiler knows which object each read is from
+    const int a_off = wave * NCS * 512 + 16 * r, h_off = S::H + (DT == Q6_K ? wave * 64 : wave * 512 + 16 * r);
+    const int b_off = S::B + q * 2048 + 16 * r, x_off = S::DX + 4 * r, s_off = S::S + r * S::SW * 2 + q * S::SW;
+
+    auto stage = [&](auto ca, auto QD, int g) __attribute__((always_inline)) {
+        constexpr int CA = decltype(ca)::value, qd = decltype(QD)::value, u = qd & 1;
+        const unsigned char* buf = u ? sb1 : sb0;
+        // this stage's own copies are in; then every wave's are, and every wave is done reading the other buffer
+        __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));   // vmcnt(0)
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if constexpr (qd < 3) issue(std::integral_constant<int, qd + 1>{}, std::integral_constant<int, 0>{});
+        else if (g + 1 < g1) issue(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+        const u32x4 ch = *reinterpret_cast<const u32x4*>(buf + (a_off + q * 512));
+        u32x4 hq = {}, hdr = {}, sv = {};
+        if constexpr (DT != Q4_K) hq = *reinterpret_cast<const u32x4*>(buf + (a_off + 1024 + q * 512));
+        if constexpr (DT == Q6_K) sv = *reinterpret_cast<const u32x4*>(buf + (a_off + 2048));
+        else hdr = *reinterpret_cast<const u32x4*>(buf + h_off);
+        const uint4 hd = make_uint4(hdr[0], hdr[1], hdr[2], hdr[3]);
+        half8 bfs[2][2];   // [step parity][K-step]
+        float dxs[2];
+        auto readb = [&](auto T) __attribute__((always_inline)) {
+            constexpr int t = decltype(T)::value, bl = t / CA, j = t % CA;
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++)
+                bfs[t & 1][ks] = *reinterpret_cast<const half8*>(buf + (b_off + (2 * bl + ks) * 4096 + j * 512));
+            dxs[t & 1] = *reinterpret_cast<const float*>(buf + (x_off + bl * 512 + j * 128));
+        };
+        readb(std::integral_constant<int, 0>{});
+        if constexpr (DT == Q6_K && qd == 0) {   // accs = −8·Σ_t sc_t·xs_t (the −32 offset, in units of 1/4), hi + lo
+            half8 ao;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const uint32_t wv = q ? (e < 4 ? sv[2] : sv[3]) : (e < 4 ? sv[0] : sv[1]);
+                ao[e] = (_Float16) (-8.0f * (float) (int8_t) ((wv >> (8 * (e & 3))) & 0xffu));
+            }
+#pragma unroll
+            for (int j = 0; j < CA; j++) {
+                const half8 shi = *reinterpret_cast<const half8*>(buf + (s_off + j * 1024));
+                const half8 slo = *reinterpret_cast<const half8*>(buf + (s_off + 4096 + j * 1024));
+                accs[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ao, shi, floatx16{}, 0, 0, 0);
+                accs[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ao, slo, accs[j], 0, 0, 0);
+            }
+        }
+        constexpr int NA = DT == Q6_K ? 4 : 2;   // weight fragments of a block: K-steps 0, 1 (Q6_K: of each plane)
+        half8 af[NA];
+        auto decode = [&](auto BL) __attribute__((always_inline)) {
+            constexpr int bl = decltype(BL)::value;
+            if constexpr (DT == Q6_K) {
+                constexpr int h2 = qd >> 1, jb = (qd & 1) + 2 * bl;   // block jb of half h2
+                const uint32_t wv = sv[2 * h2 + (jb >> 1)];
+                const float sc = (float) (int) __builtin_amdgcn_sbfe(wv, 8 * (2 * (jb & 1) + q), 8);
+                const float fm = bl ? sc * 0.015625f : sc * 0.25f, fa = bl ? -16.0f * sc : -256.0f * sc;
+                const uint32_t mul1 = pack2((_Float16) fm, (_Float16) fm), add1 = pack2((_Float16) fa, (_Float16) fa);
+                const uint32_t m1 = bl ? vmask_hi : vmask_lo;
+                af[0] = frag8(ch[0], ch[1], m1, mul1, add1);
+                af[1] = frag8(ch[2], ch[3], m1, mul1, add1);
+                const float fm2 = sc * 0.25f, fa2 = -256.0f * sc;
+                const uint32_t mul2 = pack2((_Float16) fm2, (_Float16) fm2), add2 = pack2((_Float16) fa2, (_Float16) fa2);
+                constexpr int sh = 2 * jb;   // bits 2jb..2jb+1 -> 4..5
+                auto mv = [&](uint32_t x) { return sh <= 4 ? x << (sh <= 4 ? 4 - sh : 0) : x >> (sh <= 4 ? 0 : sh - 4); };
+                af[2] = frag8(mv(hq[0]), mv(hq[1]), vmask_qh, mul2, add2);
+                af[3] = frag8(mv(hq[2]), mv(hq[3]), vmask_qh, mul2, add2);
+            } else {
+                int sci, mni;
+                q4k_scmn(hd, 2 * qd + bl, sci, mni);
+                const uint32_t sc = (uint32_t) sci;
+                // lo nibble: (1024 + v)·sc − 1024·sc; hi nibble (bits 4-7): (1024 + 16v)·sc/16 − 64·sc
+                const uint32_t dup = sc | (sc << 16) | 0x64006400u;
+                const half2v one = __builtin_bit_cast(half2v, dup) - __builtin_bit_cast(half2v, 0x64006400u);
+                const half2v mulv = bl ? one * (_Float16) 0.0625f : one;
+                const half2v addv = one * (bl ? (_Float16) -64.0f : (_Float16) -1024.0f);
+                const uint32_t mul = __builtin_bit_cast(uint32_t, mulv), add = __builtin_bit_cast(uint32_t, addv);
+                const uint32_t mask = bl ? vmask_hi : vmask_lo;
+                if constexpr (DT == Q5_K) {   // the qh byte's bit 2qd + bl is the block's fifth bit
+                    constexpr int sh = 4 * (qd >> 1);
+                    af[0] = frag8q5(ch[0], ch[1], hq[0] >> sh, hq[1] >> sh, 2 * (qd & 1) + bl, mask, mul, add);
+                    af[1] = frag8q5(ch[2], ch[3], hq[2] >> sh, hq[3] >> sh, 2 * (qd & 1) + bl, mask, mul, add);
+                } else {
+                    af[0] = frag8(ch[0], ch[1], mask, mul, add);
+                    af[1] = frag8(ch[2], ch[3], mask, mul, add);
+                }
+            }
+        };
+        // step t = (block t / CA, token tile t % CA). Its products go out between the scale FMAs of step t − 1, so that neither
+        // the second product waits for the first nor an FMA for its product; its fragments are read a step ahead.
+        floatx16 P[2];
+        auto product = [&](auto T, auto I) __attribute__((always_inline)) {
+            constexpr int t = decltype(T)::value, i = decltype(I)::value;
+            if constexpr (i == 0) P[t & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[0], bfs[t & 1][0], floatx16{}, 0, 0, 0);
+            else P[t & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bfs[t & 1][i & 1], P[t & 1], 0, 0, 0);
+        };
+        decode(std::integral_constant<int, 0>{});
+        unroll<0, NA>([&](auto I) __attribute__((always_inline)) { product(std::integral_constant<int, 0>{}, I); });
+        float x = dxs[0];
+        readb(std::integral_constant<int, 1>{});
+        unroll<0, 2 * CA>([&](auto T) __attribute__((always_inline)) {
+            constexpr int t = decltype(T)::value, bl = t / CA, j = t % CA, NE = 16 / NA;
+            const float xn = dxs[(t + 1) & 1];
+            if constexpr (t + 1 < 2 * CA && (t + 1) % CA == 0) decode(std::integral_constant<int, (t + 1) / CA>{});
+            unroll<0, NA>([&](auto I) __attribute__((always_inline)) {
+                constexpr int i = decltype(I)::value;
+                if constexpr (t + 1 < 2 * CA) product(std::integral_constant<int, t + 1>{}, I);
+                if constexpr (i == NA - 1 && t + 2 < 2 * CA) readb(std::integral_constant<int, t + 2>{});
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = NE * i; e < NE * (i + 1); e++) {
+                    if constexpr (DT != Q6_K && qd == 0 && bl == 0) accs[j][e] = P[t & 1][e] * x;
+                    else accs[j][e] = fmaf(P[t & 1][e], x, accs[j][e]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            x = xn;
+        });
+        // the stage's sums are made here: left alone, the compiler sinks their FMAs to the super-block's end, past the
+        // branches between the stages, and spills every product until then
+#pragma unroll
+        for (int j = 0; j < CA; j++) asm volatile("" : "+v"(accs[j]));
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (qd == 3) {   // super-block end: d, then (Q4_K, Q5_K) the mins on the matrix cores
+            float dds[16];
+#pragma unroll
+            for (int e = 0; e < 16; e++) {
+                const int row = 8 * (e >> 2) + 4 * q + (e & 3);
+                dds[e] = h2f_bits(*reinterpret_cast<const uint16_t*>(buf + (S::H + wave * 32 * S::HB + row * S::HB)));
+                if (DT == Q6_K) dds[e] *= 4.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < CA; j++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[j][e] = fmaf(dds[e], accs[j][e], acc[j][e]);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (DT != Q6_K) {   // A' = −dmin·mn_s for sub-blocks 4q..4q+3 of row r, split hi + lo
+                const float dmin = h2f_bits(hdr[0] >> 16);
+                half4 ahi, alo;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    int sc, mn;
+                    q4k_scmn(hd, 4 * q + e, sc, mn);
+                    const F16Pair p = split_f16(-(dmin * (float) mn));
+                    ahi[e] = p.hi;
+                    alo[e] = p.lo;
+                }
+#pragma unroll
+                for (int j = 0; j < CA; j++) {
+                    const half4 shi = *reinterpret_cast<const half4*>(buf + (s_off + j * 512));
+                    const half4 slo = *reinterpret_cast<const half4*>(buf + (s_off + 2048 + j * 512));
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x8f16(ahi, shi, acc[j], 0, 0, 0);
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x8f16(ahi, slo, acc[j], 0, 0, 0);
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x8f16(alo, shi, acc[j], 0, 0, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);   // the next stage's wait and barrier stay behind these products
+    };
+    issue(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
+    auto run = [&](auto ca) __attribute__((always_inline)) {
+        for (int g = g0; g < g1; g++) {
+            unroll<0, 4>([&](auto QD) __attribute__((always_inline)) { stage(ca, QD, g); });
+            advance();
+        }
+    };
+    if (narrow) run(std::integral_constant<int, 2>{});
+    else run(std::integral_constant<int, 4>{});
+
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int t = n0 + 32 * j + r;
+        if (t >= n || (narrow && j > 1)) continue;
+        float* ct = c + (int64_t) blockIdx.y * c_slice + (int64_t) t * ldc;
+        store_column(ct, (T0 + wave) * 32 + 4 * q, m, acc[j], A.es[t], ep, sb_per > 0);   // split K: the reduce applies the epilogue
+    }
+}
+
 // Deterministic sum of the split-K partials: c[t][row] = Σ_s part[s][t][row] in slice order.
 __global__ void __launch_bounds__(256) split_reduce_kernel(const float* __restrict__ part, int ns, int64_t slice,
                                                           int m, float* __restrict__ c, int ldc, Epi ep) {
@@ -967,11 +1253,44 @@ static hipError_t mx4_go(const WeightView& w, const GemmAct& A, int m, int n, fl
     return e != hipSuccess ? e : launch_split_reduce(part, ns, slice, m, n, c, ldc, st, ep);
 }
 
+// The wide kernel's K slices (about two workgroups per CU), or false for kq_gemm_kernel. Against it, prep and reduce included:
+// Q4_K 14336x4096 n = 512 106 / 118 us (448 tiles), n = 2048 354 / 421, n = 128 46 / 51 (112 tiles, 5 slices for 3); where it
+// needs twice the other's slices it is no faster: n = 256 70 / 68 (224), 4096x4096 n = 512 49 / 48 (128). Q6_K, bound by its
+// four products per block, gains there too: 4096x14336 n = 512 150 / 167 (128 tiles), n = 256 87 / 94 (64), 4096x4096 n = 512
+// 59 / 63.
+static bool wide_plan(int dt, int k, int m, int n, int* ns, int* sb_per) {
+    if ((dt != Q4_K && dt != Q5_K && dt != Q6_K) || n <= 64) return false;
+    const int NP = (n + 63) / 64 * 64, nsb = (k + 255) / 256, total = (m + 127) / 128 * ((NP + 127) / 128);
+    if (total < (dt == Q6_K ? 64 : NP == 128 ? 96 : 320)) return false;
+    int was, was_per;
+    split_plan((m + 127) / 128 * (NP / 64), nsb, &was, &was_per);
+    int want = total >= 320 ? 1 : (512 + total / 2) / total;
+    want = want < nsb ? want : nsb;
+    // scratch past what the other kernel's slices take must leave every allocation-free call inside its 64 MiB
+    while (want > was && gemm_act_bytes(dt, n, k) + (size_t) want * n * m * 4 > ((size_t) 60 << 20)) want--;
+    *sb_per = want > 1 ? (nsb + want - 1) / want : 0;
+    *ns = want > 1 ? (nsb + *sb_per - 1) / *sb_per : 1;
+    return true;
+}
+
+template <int DT>
+static hipError_t kq_wide_go(const WeightView& w, const GemmAct& A, int m, int n, float* c, int ldc, hipStream_t st, int ns,
+                             int sb_per, float* part, const Epi& ep) {
+    const int nrb = (m + 127) / 128, ncb = (A.NP + 127) / 128;
+    const int64_t tiles = (w.r0 + tiled_rows(m)) / 32 - w.r0 / 32, slice = (int64_t) n * m;
+    const dim3 grid((unsigned) tile_grid(false, nrb * ncb), (unsigned) ns);
+    if (ns > 1 && part == nullptr) return hipErrorInvalidValue;
+    kq_wide_kernel<DT><<<grid, MMA_THREADS, 0, st>>>(w, A, m, n, ns > 1 ? part : c, ns > 1 ? m : ldc, nrb, ncb, tiles, sb_per,
+                                                     slice, ns > 1 ? Epi{} : ep);
+    return ns > 1 ? launch_split_reduce(part, ns, slice, m, n, c, ldc, st, ep) : hipGetLastError();
+}
+
 size_t gemm_mma_split_floats(int dt, int k, int m, int n) {
     if (dt != Q4_K && dt != Q5_K && dt != Q6_K && dt != MXFP4 && dt != Q4_0 && dt != Q8_0 && dt != NVFP4 && dt != Q1_0)
         return 0;
     const int nrb = (m + 32 * MMA_WAVES - 1) / (32 * MMA_WAVES), ncb = (n + 63) / 64, nsb = (k + 255) / 256;
     int ns, sb_per;
+    if (wide_plan(dt, k, m, n, &ns, &sb_per)) return ns > 1 ? (size_t) ns * n * m : 0;
     split_plan(nrb * ncb, nsb, &ns, &sb_per);
     return ns > 1 ? (size_t) ns * n * m : 0;
 }
@@ -979,6 +1298,12 @@ size_t gemm_mma_split_floats(int dt, int k, int m, int n) {
 hipError_t launch_gemm_mma(int dt, const WeightView& w, const GemmAct& A, int k, int m, int n, float* c, int ldc,
                            hipStream_t st, float* part, const Epi& ep) {
     if (((dt == Q4_K || dt == Q5_K || dt == Q6_K) && k % 256) || (w.r0 & 31) || A.NP % 64) return hipErrorNotSupported;
+    int ns, sb_per;
+    if (wide_plan(dt, k, m, n, &ns, &sb_per)) {
+        if (dt == Q4_K) return kq_wide_go<Q4_K>(w, A, m, n, c, ldc, st, ns, sb_per, part, ep);
+        if (dt == Q5_K) return kq_wide_go<Q5_K>(w, A, m, n, c, ldc, st, ns, sb_per, part, ep);
+        return kq_wide_go<Q6_K>(w, A, m, n, c, ldc, st, ns, sb_per, part, ep);
+    }
     switch (dt) {
     case Q4_K: return kq_go<Q4_K, 1, 2>(w, A, m, n, c, ldc, st, Groups{}, part, ep);
     case Q5_K: return kq_go<Q5_K, 1, 2>(w, A, m, n, c, ldc, st, Groups{}, part, ep);
