@@ -54,33 +54,69 @@ __device__ inline float clamped_swiglu_vec(float g, float u) {
 
 // bound = the row's vector-loop bound (cols - cols % lanes, F_SPECIES.loopBound); elements past it take the
 // loop's scalar tail: SwiGLU's double formula, gpt-oss's clampedSwigluApprox. bound = 0: the full-scalar forms.
+template <int ACT> __device__ inline float glu(float g, float u, int i, int bound) {
+    if (ACT == 1) return i < bound ? silu_mul_vec(g, u) : silu_mul(g, u);
+    return ACT == 2 ? clamped_swiglu(g, u) : clamped_swiglu_vec(g, u);
+}
+
 template <int ACT>
 __global__ void __launch_bounds__(256) glu_kernel(float* __restrict__ gate, int ldg, const float* __restrict__ up,
                                                   int ldu, int rows, int cols, int bound) {
     for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
         float* g = gate + r * ldg;
         const float* u = up + r * ldu;
-        for (int i = blockIdx.x * 256 + threadIdx.x; i < cols; i += gridDim.x * 256) {
-            float v;
-            if (ACT == 1) v = i < bound ? silu_mul_vec(g[i], u[i]) : silu_mul(g[i], u[i]);
-            else if (ACT == 2) v = clamped_swiglu(g[i], u[i]);
-            else v = clamped_swiglu_vec(g[i], u[i]);
-            g[i] = v;
-        }
+        for (int i = blockIdx.x * 256 + threadIdx.x; i < cols; i += gridDim.x * 256) g[i] = glu<ACT>(g[i], u[i], i, bound);
     }
+}
+
+// Prompts: the same arithmetic on four columns per thread, rows 16-byte aligned, the pieces of all rows in one run, so that
+// no workgroup is a row's remainder. Bound by memory traffic once a thread keeps 32 bytes in flight instead of 8: gpt-oss's
+// 2048 x 2880 18.6 -> 14.6 us (71 MB, 4.8 TB/s, from the MALL), SwiGLU 512 x 14336 22.2 -> 16.6.
+template <int ACT>
+__global__ void __launch_bounds__(256) glu4_kernel(float* __restrict__ gate, int ldg, const float* __restrict__ up,
+                                                   int ldu, uint32_t pieces, uint32_t per_row, int cols, int bound) {
+    const uint32_t p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= pieces) return;
+    const int64_t r = p / per_row;
+    const int i = 4 * (int) (p % per_row);
+    float* g = gate + r * ldg + i;
+    const float* u = up + r * ldu + i;
+    if (i + 4 <= cols) {
+        const float4 x = *reinterpret_cast<const float4*>(g), y = *reinterpret_cast<const float4*>(u);
+        *reinterpret_cast<float4*>(g) = make_float4(glu<ACT>(x.x, y.x, i, bound), glu<ACT>(x.y, y.y, i + 1, bound),
+                                                    glu<ACT>(x.z, y.z, i + 2, bound), glu<ACT>(x.w, y.w, i + 3, bound));
+    } else {
+        for (int e = 0; i + e < cols; e++) g[e] = glu<ACT>(g[e], u[e], i + e, bound);
+    }
+}
+
+// Elements from which it is faster: 364 x 2880 5.3 us either way, 74 x 14336 4.9 -> 4.4, 512 x 2880 6.6 -> 5.6; below, the
+// one-column form spreads a row over more CUs.
+constexpr int64_t GLU4_MIN = 1 << 20;
+
+template <int ACT>
+static hipError_t glu_go(float* gate, int ldg, const float* up, int ldu, int rows, int cols, int bound, hipStream_t st) {
+    const int per_row = (cols + 3) / 4;
+    const int64_t pieces = (int64_t) rows * per_row;
+    const bool aligned = ((reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up)) & 15) == 0 && ldg % 4 == 0 && ldu % 4 == 0;
+    if (aligned && (int64_t) rows * cols >= GLU4_MIN && pieces <= 0x7fffffff) {
+        glu4_kernel<ACT><<<(unsigned) ((pieces + 255) / 256), 256, 0, st>>>(gate, ldg, up, ldu, (uint32_t) pieces, (uint32_t) per_row, cols, bound);
+    } else {
+        const dim3 grid((unsigned) ((cols + 255) / 256 < 64 ? (cols + 255) / 256 : 64), (unsigned) (rows < 65535 ? rows : 65535));
+        glu_kernel<ACT><<<grid, 256, 0, st>>>(gate, ldg, up, ldu, rows, cols, bound);
+    }
+    return hipGetLastError();
 }
 
 hipError_t launch_glu(int act, float* gate, int ldg, const float* up, int ldu, int rows, int cols, hipStream_t st,
                       int lanes) {
     if (rows <= 0 || cols <= 0) return hipSuccess;
     if (lanes < 0) return hipErrorInvalidValue;
-    const dim3 grid((unsigned) ((cols + 255) / 256 < 64 ? (cols + 255) / 256 : 64), (unsigned) (rows < 65535 ? rows : 65535));
     const int bound = lanes > 0 ? cols - cols % lanes : 0;
-    if (act == 1) glu_kernel<1><<<grid, 256, 0, st>>>(gate, ldg, up, ldu, rows, cols, bound);
-    else if (act == 2 && lanes == 0) glu_kernel<2><<<grid, 256, 0, st>>>(gate, ldg, up, ldu, rows, cols, 0);
-    else if (act == 2) glu_kernel<3><<<grid, 256, 0, st>>>(gate, ldg, up, ldu, rows, cols, bound);   // body = tail
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
+    if (act == 1) return glu_go<1>(gate, ldg, up, ldu, rows, cols, bound, st);
+    if (act == 2 && lanes == 0) return glu_go<2>(gate, ldg, up, ldu, rows, cols, 0, st);
+    if (act == 2) return glu_go<3>(gate, ldg, up, ldu, rows, cols, bound, st);   // body = tail
+    return hipErrorInvalidValue;
 }
 
 }  // namespace jamhip
