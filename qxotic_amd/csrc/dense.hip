@@ -449,6 +449,66 @@ __global__ void __launch_bounds__(512) dense_prep_kernel(const float* __restrict
     }
 }
 
+// Up to 64 tokens: a workgroup per token, which reads its row in whole lines; there are too few tokens for the form above to
+// fill the CUs, and its scattered reads show: F16 512x1024 n = 40 14.3 against 15.0 us, 1000x1024 n = 9 12.4 / 12.9, BF16
+// 11.5 / 11.9 (F16 of 8 to 16 tokens at k = 4096, whose largest |x| takes one wave longer here: 18.3 / 17.2).
+__global__ void __launch_bounds__(256) dense_prep_few_kernel(const float* __restrict__ a, int lda, int n, int k, int Kp,
+                                                         int NP, int hl, uint16_t* __restrict__ hi,
+                                                         uint16_t* __restrict__ lo, float* __restrict__ es) {
+    __shared__ float wmax[4];
+    const int t = blockIdx.x;
+    const float* x = a + (int64_t) t * lda;
+    float down = 1.0f;
+    if (hl) {   // the token's largest |x|; a non-finite one leaves the scale at 1 (the outputs go non-finite)
+        float mx = 0.0f;
+        for (int e = threadIdx.x; e < k; e += 256) mx = fmaxf(mx, fabsf(x[e]));
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+        if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
+        __syncthreads();
+        mx = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+        int ex;
+        if (mx > 0.0f && mx <= 3.40282347e38f) {
+            int e2;
+            frexpf(mx, &e2);   // mx in [2^(e2-1), 2^e2)
+            ex = 15 - e2;
+            ex = ex > 126 ? 126 : ex;
+        } else {
+            ex = 0;
+        }
+        down = ldexpf(1.0f, ex);
+        if (threadIdx.x == 0) es[t] = ldexpf(1.0f, -ex);
+    } else if (threadIdx.x == 0) {
+        es[t] = 1.0f;
+    }
+    // 8-element runs: run g = elements 8g..8g+7 = K-step g / 2, half g % 2
+    for (int g = threadIdx.x; g < Kp / 8; g += 256) {
+        float v[8];
+        const int e0 = 8 * g;
+        if (e0 + 8 <= k && ((reinterpret_cast<uintptr_t>(x + e0) & 15) == 0)) {
+            const float4 f0 = *reinterpret_cast<const float4*>(x + e0), f1 = *reinterpret_cast<const float4*>(x + e0 + 4);
+            v[0] = f0.x, v[1] = f0.y, v[2] = f0.z, v[3] = f0.w, v[4] = f1.x, v[5] = f1.y, v[6] = f1.z, v[7] = f1.w;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[i] = e0 + i < k ? x[e0 + i] : 0.0f;
+        }
+        uint32_t h[4], l[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            if (hl) {
+                const F16Pair p0 = split_f16(v[2 * i] * down), p1 = split_f16(v[2 * i + 1] * down);
+                h[i] = (uint32_t) __builtin_bit_cast(uint16_t, p0.hi) | ((uint32_t) __builtin_bit_cast(uint16_t, p1.hi) << 16);
+                l[i] = (uint32_t) __builtin_bit_cast(uint16_t, p0.lo) | ((uint32_t) __builtin_bit_cast(uint16_t, p1.lo) << 16);
+            } else {
+                h[i] = bf16_bits(v[2 * i]) | (bf16_bits(v[2 * i + 1]) << 16);
+            }
+        }
+        const int64_t o = ((int64_t) g * NP + t) * 8;   // (K-step g/2, half g%2) = plane row g
+        *reinterpret_cast<uint4*>(hi + o) = make_uint4(h[0], h[1], h[2], h[3]);
+        if (hl) *reinterpret_cast<uint4*>(lo + o) = make_uint4(l[0], l[1], l[2], l[3]);
+    }
+}
+
 typedef _Float16 half8d __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) void lds_void_d;
 typedef uint32_t u32x4d __attribute__((ext_vector_type(4)));
@@ -797,6 +857,8 @@ static void dense_split(int total, int nstk, int* ns, int* st_per) {
 
 // Workgroups (K slices included) from which dense_big_kernel, one per CU, beats the 128 x 64 one: 128 of them: F16 4096x14336
 // n = 512 190 against 252 us, 4096x4096 n = 256 44.5 / 51; 56 x 5 (14336x4096 n = 128) 64 / 99.
+// Not with up to 64 tokens, where half of its tile is padding: BF16 512x14336 n = 2 43.4 against 51.1 us, 1000x8192 n = 16
+// 29.0 / 33.1, F16 8000x1024 n = 12 15.1 / 17.2.
 constexpr int DBG_MIN_TILES = 128;
 
 size_t dense_mma_split_floats(int dt, int k, int m, int n) {
@@ -817,7 +879,10 @@ hipError_t launch_dense_mma(int dt, const WeightView& w, const float* a, int lda
     float* es = (float*) ((uint8_t*) scratch + pl * plane);
     // about two workgroups per CU, each with at least one pass of 64 runs
     const int ptiles = (n + 7) / 8, pmax = (Kp / 8 + 63) / 64, pwant = (512 + ptiles - 1) / ptiles;
-    dense_prep_kernel<<<dim3((unsigned) ptiles, (unsigned) (pwant < pmax ? pwant : pmax)), 512, 0, st>>>(a, lda, n, k, Kp, NP, pl == 2, xh, pl == 2 ? xl : xh, es);
+    if (n <= 64)
+        dense_prep_few_kernel<<<n, 256, 0, st>>>(a, lda, n, k, Kp, NP, pl == 2, xh, pl == 2 ? xl : xh, es);
+    else
+        dense_prep_kernel<<<dim3((unsigned) ptiles, (unsigned) (pwant < pmax ? pwant : pmax)), 512, 0, st>>>(a, lda, n, k, Kp, NP, pl == 2, xh, pl == 2 ? xl : xh, es);
     int nrb = (m + 127) / 128, ncb = NP / 64, ns, st_per;
     dense_split(nrb * ncb, Kp / DMM_STAGE, &ns, &st_per);
     if (ns > 1 && part == nullptr) return hipErrorInvalidValue;
@@ -826,7 +891,7 @@ hipError_t launch_dense_mma(int dt, const WeightView& w, const float* a, int lda
     const int64_t slice = (int64_t) n * m;
     const Epi epo = ns > 1 ? Epi{} : ep;
     const int brb = (m + 255) / 256, bcb = (NP + 127) / 128;
-    if (brb * bcb * ns >= DBG_MIN_TILES) {   // the same K slices
+    if (NP > 64 && brb * bcb * ns >= DBG_MIN_TILES) {   // the same K slices
         const dim3 grid((unsigned) tile_grid(false, brb * bcb), (unsigned) ns);
         if (pl == 2)
             dense_big_kernel<true><<<grid, 512, 0, st>>>(w, xh, xl, es, NP, Kp, k, m, n, out, ldo, brb, bcb, st_per, slice, epo);
