@@ -123,12 +123,15 @@ struct GemmAct {
     const _Float16* shi;   // per-32 sums (Q4_K, Q4_0) [Kp/256][NP][8] or per-16 sums (Q6_K) [Kp/256][NP][16],
     const _Float16* slo;   //   · 2^-e_t, split as f16 high part + f16 remainder
     const float* es;       // [NP] 2^e_t
-    // MXFP4 (mx4.hip): b holds the first 16 bytes and b8 the last 8 of each block's 32 high (0) or low (1) digits, 6
-    // bits each in the order of the weights' nibbles, [Kp/32][2][NP][16 B] and [..][8 B]; dx is [Kp/128][NP][4]
-    const uint8_t* b8;
+    // MXFP4 (mx4.hip): b holds the first 16 bytes of each block's 32 high (0) or low (1) digits, 6 bits each in the order of
+    // the weights' nibbles, [Kp/32][2][NP][16 B], and after these (Kp·NP bytes in) the last 8, [Kp/32][2][NP][8 B]; dx is
+    // [Kp/128][NP][4]
     int NP, Kp;
     int K;                 // the call's k (blocks past it are zero)
 };
+// An argument of every prefill kernel: with 8 bytes more (one type's pointer) the same instructions ran 1 to 3% longer on
+// calls of a few tens of microseconds (Q4_K 14336x4096 n = 9 21.3 against 20.65 us, Q8_0 2880x4096 n = 77 23.4 / 23.2).
+static_assert(sizeof(GemmAct) == 56, "GemmAct grew");
 int gemm_sums_kind(int dt);   // 0 none, 1 per-32 sums, 2 per-16 sums
 size_t gemm_act_bytes(int dt, int n, int k);
 bool gemm_prep_fits(int k);

@@ -117,7 +117,7 @@ __global__ void __launch_bounds__(64 * mx4::WAVES, 2) mx4_gemm_kernel(WeightView
     for (int i = 0; i < RT; i++) a_src[i] = w.qs + tile(TL + i) * G * (NC * CHUNK_STRIDE) + 16 * lane;
     const uint8_t* h_src = w.sc + (tile(TL + (RT == 2 ? q : 0)) * G * 32 + r) * 16;
     const uint8_t* b16_src = reinterpret_cast<const uint8_t*>(A.b) + ((int64_t) (2 * wave) * A.NP + n0 + lane) * 16;
-    const uint8_t* b8_src = A.b8 + ((int64_t) (2 * wave + q) * A.NP + n0) * 8 + 16 * r;
+    const uint8_t* b8_src = reinterpret_cast<const uint8_t*>(A.b) + (int64_t) A.Kp * A.NP + ((int64_t) (2 * wave + q) * A.NP + n0) * 8 + 16 * r;
     const float* dx_src = A.dx + ((int64_t) n0 + lane) * 4;
     const int64_t np = A.NP;
     auto issue = [&](int st, unsigned char* buf) {

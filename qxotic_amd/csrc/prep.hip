@@ -225,7 +225,7 @@ constexpr int PREP_GRID = 1024;      // a multiple of 8 (XCDs)
 // MXO: the MXFP4 element order (a weight byte's two nibbles are elements e and e + 16 of the block).
 // ORD: the element order of the codes inside a K-step, matching the weight operand the GEMM builds:
 //   0  elements 16q + 8ks + perm8(i)            (nibble / byte fields, Q4_K, Q5_K, Q6_K, Q4_0, Q8_0, Q1_0)
-//   1  pairs (e, e + 16) of the 32-block, as two 6-bit digits per code (MXFP4; GemmAct::b8)
+//   1  pairs (e, e + 16) of the 32-block, as two 6-bit digits per code (MXFP4; GemmAct::b)
 //   2  pairs (u, u + 8) of each 16-element sub-block, K-step ks = sub-block ks of the block (NVFP4)
 // f1all: jam's F1 quantization for every slot (NVFP4, whose only jam path is F1 at every n, jam.c:662-668).
 template <int SK, int ORD, int SG>
@@ -484,7 +484,7 @@ static hipError_t prep_np(int dt, const float* a, int lda, int n, int NP, int k,
     _Float16* slo = (_Float16*) (p + sb);
     p += 2 * sb;
     float* es = (float*) p;
-    *out = GemmAct{bq, dx, shi, slo, es, (const uint8_t*) bq + (int64_t) Kp * NP, NP, Kp, k};
+    *out = GemmAct{bq, dx, shi, slo, es, NP, Kp, k};
     if (NP <= 0) return hipSuccess;
     const int vec = ((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (lda & 3) == 0) ? 1 : 0;
     const int kind = dt == MXFP4 ? 3 : dt == NVFP4 ? 4 : sk;
