@@ -217,17 +217,20 @@ __global__ void __launch_bounds__(64 * DG_WAVES) dense_gemv2_kernel(WeightView w
         load(raw[1], j + 3 * JS);
     }
     if constexpr (KS) {   // every wave reaches this: row0 < m for the whole workgroup
-        __shared__ float part[DG_WAVES][NT];
+        // the waves' sums [DG_WAVES][NT] take the activations' place: beside a full 64 KB of them a launch would ask for
+        // more LDS than it may without raising its kernel's limit
+        static_assert(DG_WAVES <= 64 * V, "the sums fit the shortest activation rows");
+        __syncthreads();   // every wave is done with the activations
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             const float v = wave_sum(acc[0][t]);
-            if (lane == 0) part[wave][t] = v;
+            if (lane == 0) xs[wave * NT + t] = v;
         }
         __syncthreads();
         if ((int) threadIdx.x < ntv) {
             const int t = threadIdx.x;
             float* dst = c + (int64_t) (t0 + t) * ldc + row0;
-            *dst = epilogue(ep, (part[0][t] + part[1][t]) + (part[2][t] + part[3][t]), row0, dst);
+            *dst = epilogue(ep, (xs[t] + xs[NT + t]) + (xs[2 * NT + t] + xs[3 * NT + t]), row0, dst);
         }
         return;
     }

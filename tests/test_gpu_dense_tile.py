@@ -29,6 +29,9 @@ def test_short_dense(hip, dt, m, n, k):
         w, w64 = wt.view(torch.uint8).numpy(), wt.double().numpy()
         rounds = (n >= 8 and k % 2 == 0) or k % 32 == 0   # jam.c:622-652
         x64 = (torch.from_numpy(a).bfloat16().double().numpy()) if rounds else a.astype(np.float64)
+    elif dt == O.F16:
+        wt = w32.astype(np.float16)
+        w, w64, x64 = wt, wt.astype(np.float64), a.astype(np.float64)
     else:
         w, w64, x64 = w32, w32.astype(np.float64), a.astype(np.float64)
     ref, bound = x64 @ w64.T, (k + 2) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T)
@@ -51,6 +54,13 @@ def test_short_dense(hip, dt, m, n, k):
             assert (np.abs(fused - whole) <= bound + 2.0 ** -23 * (np.abs(ref) + np.abs(bias) + np.abs(c0))).all()
     finally:
         hip.evict(Segment.of(w))
+
+
+# a workgroup per row whose activations fill the 64 KB of LDS, and one row beside that
+@pytest.mark.parametrize("m,n,k", [(128, 8, 2048), (256, 4, 4096), (1, 5, 2048), (255, 3, 4001)])
+@pytest.mark.parametrize("dt", [O.F32, O.F16, O.BF16])
+def test_row_split_full_lds(hip, dt, m, n, k):
+    test_short_dense(hip, dt, m, n, k)
 
 
 # n past 64 with enough tiles: 256 x 128 workgroups, 64 of k per stage; whole, split and masked last stages, ragged edges
