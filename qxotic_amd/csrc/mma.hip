@@ -30,6 +30,7 @@
 // weight tile is read from HBM into that XCD's L2 once.
 #include "common.h"
 #include "launch.h"
+#include "plan.h"
 
 #include <atomic>
 #include <type_traits>
@@ -1170,19 +1171,6 @@ hipError_t launch_split_reduce(const float* part, int ns, int64_t slice, int m, 
     return hipGetLastError();
 }
 
-// K slices for a grid of `total` workgroups: enough for about two workgroups per CU, whole super-blocks each.
-static void split_plan(int total, int nsb, int* ns, int* sb_per) {
-    int want = total >= 384 ? 1 : (512 + total - 1) / total;
-    want = want < nsb ? want : nsb;
-    *sb_per = want > 1 ? (nsb + want - 1) / want : 0;
-    *ns = want > 1 ? (nsb + *sb_per - 1) / *sb_per : 1;
-}
-
-// Workgroups of two resident per CU take about the same CU time whether a CU holds one or two, so a call
-// takes ceil(tiles per CU) tile times: Q4_K 14336x4096 at n = 448, 512 and 576 (784, 896 and 1008 tiles)
-// all ran 128 us. Each XCD takes a contiguous run of T8 = ceil(tiles / 8) tiles over its CUs; when that
-// leaves r <= CUs / 2 tiles for a last partial round, those r tiles run as 2r half tiles (32 tokens) instead,
-// one per CU. Returns r, or 0 for no split.
 // CUs per device, filled by gemm_tail_prime at context creation (before any caller can be capturing a graph)
 static std::atomic<int> g_cus[64];
 void gemm_tail_prime(int dev) {
@@ -1195,14 +1183,7 @@ int device_cus() {
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
     return g_cus[dev].load(std::memory_order_relaxed);
 }
-static int tail_split(int total) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-    const int n = g_cus[dev].load(std::memory_order_relaxed);
-    if (n < 8) return 0;   // not primed: no split
-    const int cu8 = n / 8, T8 = (total + 7) / 8, r = T8 % cu8;
-    return r > 0 && 2 * r <= cu8 ? r : 0;
-}
+static int tail_split(int total) { return tail_tiles(total, device_cus()); }
 
 template <int DT, int RT, int CT>
 static hipError_t kq_go(const WeightView& w, const GemmAct& A, int m, int n, float* c, int ldc, hipStream_t st,
@@ -1219,18 +1200,17 @@ static hipError_t kq_go(const WeightView& w, const GemmAct& A, int m, int n, flo
         if (e != hipSuccess) return e;
         attr.store(true, std::memory_order_release);
     }
-    int ns = 1, sb_per = 0;
-    if (part != nullptr) split_plan(total, A.Kp / 256, &ns, &sb_per);
-    if (ns == 1) {
+    const Split sp = part != nullptr ? split_plan(total, A.Kp / 256) : Split{1, 0};
+    if (sp.ns == 1) {
         const int xs = gp.map64 == nullptr ? tail_split(total) : 0;
         kq_gemm_kernel<DT, RT, CT><<<grid + 8 * xs, MMA_THREADS, lds, st>>>(w, A, m, n, c, ldc, nrb, ncb, tiles, gp, 0,
                                                                             0, ep, xs);
         return hipGetLastError();
     }
     const int64_t slice = (int64_t) n * m;
-    kq_gemm_kernel<DT, RT, CT><<<dim3(grid, ns), MMA_THREADS, lds, st>>>(w, A, m, n, part, m, nrb, ncb, tiles, gp,
-                                                                         sb_per, slice, Epi{}, 0);
-    split_reduce_kernel<<<dim3((m + 255) / 256, n), 256, 0, st>>>(part, ns, slice, m, c, ldc, ep);
+    kq_gemm_kernel<DT, RT, CT><<<dim3(grid, sp.ns), MMA_THREADS, lds, st>>>(w, A, m, n, part, m, nrb, ncb, tiles, gp,
+                                                                            sp.per, slice, Epi{}, 0);
+    split_reduce_kernel<<<dim3((m + 255) / 256, n), 256, 0, st>>>(part, sp.ns, slice, m, c, ldc, ep);
     return hipGetLastError();
 }
 
@@ -1245,64 +1225,43 @@ static int mx4_rt(int m, int k, int ncb) {
 static hipError_t mx4_go(const WeightView& w, const GemmAct& A, int m, int n, float* c, int ldc, hipStream_t st, float* part,
                          const Epi& ep) {
     const int ncb = A.NP / 64, rt = mx4_rt(m, A.K, ncb), total = (m + 128 * rt - 1) / (128 * rt) * ncb;
-    int ns = 1, sb_per = 0;
-    if (rt == 1 && part != nullptr) split_plan(total, A.Kp / 256, &ns, &sb_per);
-    if (ns == 1) return launch_mx4_gemm(w, A, m, n, c, ldc, st, Groups{}, rt, 1, 0, tail_split(total), 0, ep);
+    const Split sp = rt == 1 && part != nullptr ? split_plan(total, A.Kp / 256) : Split{1, 0};
+    if (sp.ns == 1) return launch_mx4_gemm(w, A, m, n, c, ldc, st, Groups{}, rt, 1, 0, tail_split(total), 0, ep);
     const int64_t slice = (int64_t) n * m;
-    const hipError_t e = launch_mx4_gemm(w, A, m, n, part, m, st, Groups{}, rt, ns, sb_per, 0, slice, Epi{});
-    return e != hipSuccess ? e : launch_split_reduce(part, ns, slice, m, n, c, ldc, st, ep);
+    const hipError_t e = launch_mx4_gemm(w, A, m, n, part, m, st, Groups{}, rt, sp.ns, sp.per, 0, slice, Epi{});
+    return e != hipSuccess ? e : launch_split_reduce(part, sp.ns, slice, m, n, c, ldc, st, ep);
 }
 
-// The wide kernel's K slices (about two workgroups per CU), or false for kq_gemm_kernel. Against it, prep and reduce included:
-// Q4_K 14336x4096 n = 512 106 / 118 us (448 tiles), n = 2048 354 / 421, n = 128 46 / 51 (112 tiles, 5 slices for 3); where it
-// needs twice the other's slices it is no faster: n = 256 70 / 68 (224), 4096x4096 n = 512 49 / 48 (128). Q6_K, bound by its
-// four products per block, gains there too: 4096x14336 n = 512 150 / 167 (128 tiles), n = 256 87 / 94 (64), 4096x4096 n = 512
-// 59 / 63.
-static bool wide_plan(int dt, int k, int m, int n, int* ns, int* sb_per) {
-    if ((dt != Q4_K && dt != Q5_K && dt != Q6_K) || n <= 64) return false;
-    const int NP = (n + 63) / 64 * 64, nsb = (k + 255) / 256, total = (m + 127) / 128 * ((NP + 127) / 128);
-    if (total < (dt == Q6_K ? 64 : NP == 128 ? 96 : 320)) return false;
-    int was, was_per;
-    split_plan((m + 127) / 128 * (NP / 64), nsb, &was, &was_per);
-    int want = total >= 320 ? 1 : (512 + total / 2) / total;
-    want = want < nsb ? want : nsb;
-    // scratch past what the other kernel's slices take must leave every allocation-free call inside its 64 MiB
-    while (want > was && gemm_act_bytes(dt, n, k) + (size_t) want * n * m * 4 > ((size_t) 60 << 20)) want--;
-    *sb_per = want > 1 ? (nsb + want - 1) / want : 0;
-    *ns = want > 1 ? (nsb + *sb_per - 1) / *sb_per : 1;
-    return true;
-}
+static WidePlan wide_of(int dt, int k, int m, int n) { return wide_plan(dt, k, m, n, device_cus(), gemm_act_bytes(dt, n, k)); }
 
 template <int DT>
-static hipError_t kq_wide_go(const WeightView& w, const GemmAct& A, int m, int n, float* c, int ldc, hipStream_t st, int ns,
-                             int sb_per, float* part, const Epi& ep) {
+static hipError_t kq_wide_go(const WeightView& w, const GemmAct& A, int m, int n, float* c, int ldc, hipStream_t st, Split sp,
+                             float* part, const Epi& ep) {
     const int nrb = (m + 127) / 128, ncb = (A.NP + 127) / 128;
     const int64_t tiles = (w.r0 + tiled_rows(m)) / 32 - w.r0 / 32, slice = (int64_t) n * m;
-    const dim3 grid((unsigned) tile_grid(false, nrb * ncb), (unsigned) ns);
-    if (ns > 1 && part == nullptr) return hipErrorInvalidValue;
-    kq_wide_kernel<DT><<<grid, MMA_THREADS, 0, st>>>(w, A, m, n, ns > 1 ? part : c, ns > 1 ? m : ldc, nrb, ncb, tiles, sb_per,
-                                                     slice, ns > 1 ? Epi{} : ep);
-    return ns > 1 ? launch_split_reduce(part, ns, slice, m, n, c, ldc, st, ep) : hipGetLastError();
+    const dim3 grid((unsigned) tile_grid(false, nrb * ncb), (unsigned) sp.ns);
+    if (sp.ns > 1 && part == nullptr) return hipErrorInvalidValue;
+    kq_wide_kernel<DT><<<grid, MMA_THREADS, 0, st>>>(w, A, m, n, sp.ns > 1 ? part : c, sp.ns > 1 ? m : ldc, nrb, ncb, tiles,
+                                                     sp.per, slice, sp.ns > 1 ? Epi{} : ep);
+    return sp.ns > 1 ? launch_split_reduce(part, sp.ns, slice, m, n, c, ldc, st, ep) : hipGetLastError();
 }
 
 size_t gemm_mma_split_floats(int dt, int k, int m, int n) {
     if (dt != Q4_K && dt != Q5_K && dt != Q6_K && dt != MXFP4 && dt != Q4_0 && dt != Q8_0 && dt != NVFP4 && dt != Q1_0)
         return 0;
-    const int nrb = (m + 32 * MMA_WAVES - 1) / (32 * MMA_WAVES), ncb = (n + 63) / 64, nsb = (k + 255) / 256;
-    int ns, sb_per;
-    if (wide_plan(dt, k, m, n, &ns, &sb_per)) return ns > 1 ? (size_t) ns * n * m : 0;
-    split_plan(nrb * ncb, nsb, &ns, &sb_per);
+    const WidePlan wp = wide_of(dt, k, m, n);
+    const int ns = wp.wide ? wp.k.ns : split_plan(up_div(m, 32 * MMA_WAVES) * up_div(n, 64), up_div(k, 256)).ns;
     return ns > 1 ? (size_t) ns * n * m : 0;
 }
 
 hipError_t launch_gemm_mma(int dt, const WeightView& w, const GemmAct& A, int k, int m, int n, float* c, int ldc,
                            hipStream_t st, float* part, const Epi& ep) {
     if (((dt == Q4_K || dt == Q5_K || dt == Q6_K) && k % 256) || (w.r0 & 31) || A.NP % 64) return hipErrorNotSupported;
-    int ns, sb_per;
-    if (wide_plan(dt, k, m, n, &ns, &sb_per)) {
-        if (dt == Q4_K) return kq_wide_go<Q4_K>(w, A, m, n, c, ldc, st, ns, sb_per, part, ep);
-        if (dt == Q5_K) return kq_wide_go<Q5_K>(w, A, m, n, c, ldc, st, ns, sb_per, part, ep);
-        return kq_wide_go<Q6_K>(w, A, m, n, c, ldc, st, ns, sb_per, part, ep);
+    const WidePlan wp = wide_of(dt, k, m, n);
+    if (wp.wide) {
+        if (dt == Q4_K) return kq_wide_go<Q4_K>(w, A, m, n, c, ldc, st, wp.k, part, ep);
+        if (dt == Q5_K) return kq_wide_go<Q5_K>(w, A, m, n, c, ldc, st, wp.k, part, ep);
+        return kq_wide_go<Q6_K>(w, A, m, n, c, ldc, st, wp.k, part, ep);
     }
     switch (dt) {
     case Q4_K: return kq_go<Q4_K, 1, 2>(w, A, m, n, c, ldc, st, Groups{}, part, ep);

@@ -1,0 +1,81 @@
+// Which kernel of a family takes a call and how it splits k: plain arithmetic on the call's sizes, shared by the launchers,
+// by the sizing of their scratch and by the tests (compiles without HIP).
+#pragma once
+
+#include <stddef.h>
+#include <stdint.h>
+
+#include "dtype.h"
+
+namespace jamhip {
+
+inline int up_div(int a, int b) { return (a + b - 1) / b; }
+
+// K slices of a matrix-core GEMM: ns of them, `per` K units each (0 when whole).
+struct Split {
+    int ns, per;
+};
+
+// K slices for a grid of `total` workgroups: enough for about two workgroups per CU, whole units each.
+inline Split split_plan(int total, int units) {
+    int want = total >= 384 ? 1 : up_div(512, total);
+    want = want < units ? want : units;
+    const int per = want > 1 ? up_div(units, want) : 0;
+    return {want > 1 ? up_div(units, per) : 1, per};
+}
+
+// Workgroups of two resident per CU take about the same CU time whether a CU holds one or two, so a call
+// takes ceil(tiles per CU) tile times: Q4_K 14336x4096 at n = 448, 512 and 576 (784, 896 and 1008 tiles)
+// all ran 128 us. Each XCD takes a contiguous run of T8 = ceil(tiles / 8) tiles over its CUs; when that
+// leaves r <= CUs / 2 tiles for a last partial round, those r tiles run as 2r half tiles (32 tokens) instead,
+// one per CU. Returns r, or 0 for no split.
+inline int tail_tiles(int total, int cus) {
+    if (cus < 8) return 0;   // not primed: no split
+    const int cu8 = cus / 8, r = up_div(total, 8) % cu8;
+    return r > 0 && 2 * r <= cu8 ? r : 0;
+}
+
+// Half tiles that the fullest CU computes, for `total` tiles times `ns` K slices.
+inline int cu_half_tiles(int total, int ns, int cus, bool tail) {
+    const int cu8 = cus < 8 ? 32 : cus / 8, t8 = up_div(total, 8) * ns, r = t8 % cu8;
+    return 2 * (t8 / cu8) + (r == 0 ? 0 : tail && 2 * r <= cu8 ? 1 : 2);
+}
+
+// The K-quants past 64 tokens: kq_wide_kernel (128 x 128 tiles), or kq_gemm_kernel (128 x 64). Both leave CUs idle in their
+// last round, at different sizes, so neither is the faster one from some size on; the rule compares what the fullest CU has
+// to do, in super-block times of a 128 x 64 tile. A wide tile takes 1.6 of them (one half of it padding or not), its longer
+// start and end 3, and each million floats of split-K partials 0.3. Both kernels with prep and reduce, in us:
+//   Q4_K 14336x4096 n = 512 (448 wide tiles, 2 rounds, against 3.5) 103 / 111; n = 576 (560, 3 against 4) 137 / 120;
+//   n = 260 (336, 2 against 2.5) 92 / 83; n = 2048 366 / 433; 28672x4096 n = 260 161 / 134; 12288x4096 n = 384 93 / 87;
+//   16384x1024 n = 65 (1 super-block per slice) 27.8 / 22.5; Q5_K 14336x4096 n = 576 152 / 140; Q6_K 4096x14336 n = 512
+//   (128 tiles, 4 slices for 2) 153 / 168, n = 129 76 / 72; 12288x4096 n = 260 107 / 87; 16384x1024 n = 129 (2 slices for 1) 1.4 : 1.
+// Over 867 such points (14 shapes, 65 to 2048 tokens) no call that goes to the wide kernel was over 1.1% behind the other.
+// Two exceptions are in it: Q4_K, the lightest to decode, is not split where kq_gemm_kernel is whole, nor whole where the
+// scratch left no room to split (4096x14336 n = 1024, 256 workgroups, 242 / 227), and three blocks of 64 tokens, padded to
+// four, are not split finer past 4 slices (Q6_K 4096x14336 n = 129, above, 8 slices for 6).
+struct WidePlan {
+    bool wide;
+    Split k;
+};
+inline WidePlan wide_plan(int dt, int k, int m, int n, int cus, size_t act_bytes) {
+    if ((dt != Q4_K && dt != Q5_K && dt != Q6_K) || n <= 64) return {false, {1, 0}};
+    const int NP = up_div(n, 64) * 64, nsb = up_div(k, 256), rows = up_div(m, 128);
+    const int total = rows * up_div(NP, 128), ototal = rows * (NP / 64);
+    const Split o = split_plan(ototal, nsb);
+    // about two workgroups per CU
+    int want = total >= 320 ? 1 : (512 + total / 2) / total;
+    want = want < nsb ? want : nsb;
+    // scratch past what the other kernel's slices take must leave every allocation-free call inside its 64 MiB
+    while (want > o.ns && act_bytes + (size_t) want * n * m * 4 > ((size_t) 60 << 20)) want--;
+    Split s{1, 0};
+    if (want > 1) s.per = up_div(nsb, want), s.ns = up_div(nsb, s.per);
+    const bool split = s.ns > 1, osplit = o.ns > 1;
+    if (dt == Q4_K && (split ? !osplit : total < 320)) return {false, {1, 0}};
+    if (NP == 192 && s.ns > o.ns && s.ns > 4) return {false, {1, 0}};
+    const double part = 0.3e-6 * n * m;
+    const double wide = 1.6 * (split ? s.per : nsb) * cu_half_tiles(total, s.ns, cus, false) / 2 + (split ? s.ns * part : 0) + 3;
+    const double other = (double) (osplit ? o.per : nsb) * cu_half_tiles(ototal, o.ns, cus, !osplit) / 2 + (osplit ? o.ns * part : 0);
+    return {wide < other, s};
+}
+
+}  // namespace jamhip

@@ -1,0 +1,82 @@
+"""The rules that choose a kernel and its K slices (csrc/plan.h), on the CPU: at sizes where both kernels were measured the
+rule takes the faster one, over the whole range it stays within what the kernels and the scratch can hold."""
+import ctypes
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from oracle import oracle as O
+
+CSRC = Path(__file__).resolve().parent.parent / "qxotic_amd" / "csrc"
+SHIM = """
+#include "plan.h"
+using namespace jamhip;
+extern "C" void q_wide(int dt, int k, int m, int n, size_t act, int* o) {
+    const WidePlan p = wide_plan(dt, k, m, n, 256, act);
+    o[0] = p.wide, o[1] = p.k.ns, o[2] = p.k.per;
+}
+extern "C" void q_split(int total, int units, int* o) { const Split s = split_plan(total, units); o[0] = s.ns, o[1] = s.per; }
+extern "C" int q_tail(int total, int cus) { return tail_tiles(total, cus); }
+"""
+
+
+class Plans:
+    def __init__(self, so):
+        self.lib = ctypes.CDLL(str(so))
+
+    def _get(self, name, size, *args):
+        o = (ctypes.c_int * size)()
+        getattr(self.lib, name)(*args, o)
+        return list(o)
+
+    def wide(self, dt, k, m, n):
+        np_, sums = (n + 63) // 64 * 64, 16 if dt == O.Q6_K else 8
+        act = k * np_ * 2 + k // 32 * np_ * 4 + 2 * (k // 256 * np_ * sums * 2) + 4 * np_
+        return self._get("q_wide", 3, dt, k, m, n, ctypes.c_size_t(act))
+
+    def split(self, total, units):
+        return self._get("q_split", 2, total, units)
+
+
+@pytest.fixture(scope="session")
+def plans(tmp_path_factory):
+    d = tmp_path_factory.mktemp("plans")
+    (d / "plans.cpp").write_text(SHIM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{CSRC}", str(d / "plans.cpp"), "-o",
+                    str(d / "plans.so")], check=True)
+    return Plans(d / "plans.so")
+
+
+# (type, m, k, n, the wide kernel is the faster one), measured with prep and reduce; every pair differs by 4% or more
+WIDE = [(O.Q4_K, 14336, 4096, 512, True), (O.Q4_K, 14336, 4096, 2048, True), (O.Q4_K, 14336, 4096, 128, True),
+        (O.Q4_K, 14336, 4096, 260, False), (O.Q4_K, 14336, 4096, 576, False), (O.Q4_K, 28672, 4096, 128, False),
+        (O.Q4_K, 28672, 4096, 260, False), (O.Q4_K, 16384, 1024, 65, False), (O.Q4_K, 128256, 1024, 160, False),
+        (O.Q4_K, 128256, 1024, 96, True), (O.Q4_K, 4096, 14336, 1024, False), (O.Q4_K, 4096, 14336, 384, True),
+        (O.Q5_K, 14336, 4096, 260, False), (O.Q5_K, 14336, 4096, 576, False), (O.Q5_K, 8192, 4096, 576, False),
+        (O.Q5_K, 14336, 4096, 512, True), (O.Q6_K, 4096, 14336, 512, True), (O.Q6_K, 14336, 4096, 129, False),
+        (O.Q6_K, 12288, 4096, 260, False), (O.Q6_K, 12288, 4096, 160, False), (O.Q6_K, 8192, 4096, 384, False),
+        (O.Q6_K, 4096, 4096, 160, False), (O.Q6_K, 16384, 1024, 160, False), (O.Q6_K, 4096, 14336, 129, False),
+        (O.Q6_K, 14336, 4096, 512, True)]
+
+
+@pytest.mark.parametrize("dt,m,k,n,wide", WIDE)
+def test_wide_where_it_is_faster(plans, dt, m, k, n, wide):
+    assert plans.wide(dt, k, m, n)[0] == wide
+
+
+@pytest.mark.parametrize("dt", [O.Q4_K, O.Q5_K, O.Q6_K])
+def test_wide_slices(plans, dt):
+    """Whole super-blocks that cover k, none of the slices empty, and no more scratch than the 64 MiB of an allocation-free
+    call unless the other kernel's slices take it too."""
+    for m in (1, 128, 129, 1000, 4096, 14336, 128256):
+        for nsb in (1, 2, 5, 16, 56):
+            for n in (65, 128, 129, 200, 512, 4150):
+                wide, ns, per = plans.wide(dt, 256 * nsb, m, n)
+                if not wide:
+                    continue
+                assert (ns, per) == (1, 0) or (per * (ns - 1) < nsb <= per * ns)
+                other = plans.split((m + 127) // 128 * ((n + 63) // 64), nsb)[0]
+                assert ns <= max(1, other) or ns * n * m * 4 <= 60 << 20
+    assert not any(plans.wide(dt, 4096, 14336, n)[0] for n in (1, 9, 64))
+    assert not plans.wide(O.Q8_0, 4096, 14336, 512)[0]
