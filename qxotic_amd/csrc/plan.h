@@ -53,6 +53,9 @@ inline int cu_half_tiles(int total, int ns, int cus, bool tail) {
 // Two exceptions are in it: Q4_K, the lightest to decode, is not split where kq_gemm_kernel is whole, nor whole where the
 // scratch left no room to split (4096x14336 n = 1024, 256 workgroups, 242 / 227), and three blocks of 64 tokens, padded to
 // four, are not split finer past 4 slices (Q6_K 4096x14336 n = 129, above, 8 slices for 6).
+// kq_wide_kernel addresses a super-block's codes and the next one's first by 32-bit offsets: up to 11 blocks of 64 bytes a
+// token, which pass 2^32 at 6.1 million.
+constexpr int WIDE_MAX_TOKENS = 1 << 22;
 struct WidePlan {
     bool wide;
     Split k;
@@ -60,6 +63,7 @@ struct WidePlan {
 inline WidePlan wide_plan(int dt, int k, int m, int n, int cus, size_t act_bytes) {
     if ((dt != Q4_K && dt != Q5_K && dt != Q6_K) || n <= 64) return {false, {1, 0}};
     const int NP = up_div(n, 64) * 64, nsb = up_div(k, 256), rows = up_div(m, 128);
+    if (NP > WIDE_MAX_TOKENS) return {false, {1, 0}};
     const int total = rows * up_div(NP, 128), ototal = rows * (NP / 64);
     const Split o = split_plan(ototal, nsb);
     // about two workgroups per CU

@@ -80,3 +80,11 @@ def test_wide_slices(plans, dt):
                 assert ns <= max(1, other) or ns * n * m * 4 <= 60 << 20
     assert not any(plans.wide(dt, 4096, 14336, n)[0] for n in (1, 9, 64))
     assert not plans.wide(O.Q8_0, 4096, 14336, 512)[0]
+
+
+def test_wide_offsets_fit_32_bits(plans):
+    """The wide kernel reads token slot t of block b (up to 10: the next super-block's first stage) at the 32-bit offset
+    b * 64 * slots + 16 * t from its super-block: longer calls stay with the other kernel."""
+    most = max(n for n in (1 << 16, 1 << 20, (1 << 22) - 64, 1 << 22, (1 << 22) + 1, 5 << 20, 1 << 23, 1 << 24)
+               if plans.wide(O.Q6_K, 256, 512, n)[0])
+    assert 11 * 64 * ((most + 63) // 64 * 64) < 1 << 32
