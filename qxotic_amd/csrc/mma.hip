@@ -1214,22 +1214,15 @@ static hipError_t kq_go(const WeightView& w, const GemmAct& A, int m, int n, flo
     return hipGetLastError();
 }
 
-// MXFP4 (mx4.hip): waves of 64 rows (256-row workgroups, k whole) once those give each CU one, or at k <= 4096, where a
-// whole k is short, once they give every third CU one; else waves of 32 rows with the K split of the other types.
-// 64 against 32 rows: 14336x4096 n = 320 55.7 / 67.2 us (280 workgroups), n = 512 72.8 / 80.1, n = 128 36.5 / 38.8 (112),
-// 5760x2880 n = 256 27.5 / 32.0 (92), n = 512 37.9 / 41.8; but 14336x4096 n = 64 34.4 / 24.7 (56), 4096x14336 n = 512 111 /
-// 84 (128). A whole k of 64-row waves split like the others measures as the 32-row waves do.
-static int mx4_rt(int m, int k, int ncb) {
-    return m >= 512 && (m + 255) / 256 * ncb >= (k <= 4096 ? 88 : 256) ? 2 : 1;
-}
+// MXFP4 (mx4.hip) under mx4_plan.
 static hipError_t mx4_go(const WeightView& w, const GemmAct& A, int m, int n, float* c, int ldc, hipStream_t st, float* part,
                          const Epi& ep) {
-    const int ncb = A.NP / 64, rt = mx4_rt(m, A.K, ncb), total = (m + 128 * rt - 1) / (128 * rt) * ncb;
-    const Split sp = rt == 1 && part != nullptr ? split_plan(total, A.Kp / 256) : Split{1, 0};
-    if (sp.ns == 1) return launch_mx4_gemm(w, A, m, n, c, ldc, st, Groups{}, rt, 1, 0, tail_split(total), 0, ep);
+    const Mx4Plan p = mx4_plan(m, A.K, n);
+    if (p.k.ns == 1 || part == nullptr)
+        return launch_mx4_gemm(w, A, m, n, c, ldc, st, Groups{}, p.rt, 1, 0, tail_split(p.tiles), 0, ep);
     const int64_t slice = (int64_t) n * m;
-    const hipError_t e = launch_mx4_gemm(w, A, m, n, part, m, st, Groups{}, rt, sp.ns, sp.per, 0, slice, Epi{});
-    return e != hipSuccess ? e : launch_split_reduce(part, sp.ns, slice, m, n, c, ldc, st, ep);
+    const hipError_t e = launch_mx4_gemm(w, A, m, n, part, m, st, Groups{}, p.rt, p.k.ns, p.k.per, 0, slice, Epi{});
+    return e != hipSuccess ? e : launch_split_reduce(part, p.k.ns, slice, m, n, c, ldc, st, ep);
 }
 
 static WidePlan wide_of(int dt, int k, int m, int n) { return wide_plan(dt, k, m, n, device_cus(), gemm_act_bytes(dt, n, k)); }
@@ -1237,10 +1230,10 @@ static WidePlan wide_of(int dt, int k, int m, int n) { return wide_plan(dt, k, m
 template <int DT>
 static hipError_t kq_wide_go(const WeightView& w, const GemmAct& A, int m, int n, float* c, int ldc, hipStream_t st, Split sp,
                              float* part, const Epi& ep) {
+    if (part == nullptr) sp = {1, 0};
     const int nrb = (m + 127) / 128, ncb = (A.NP + 127) / 128;
     const int64_t tiles = (w.r0 + tiled_rows(m)) / 32 - w.r0 / 32, slice = (int64_t) n * m;
     const dim3 grid((unsigned) tile_grid(false, nrb * ncb), (unsigned) sp.ns);
-    if (sp.ns > 1 && part == nullptr) return hipErrorInvalidValue;
     kq_wide_kernel<DT><<<grid, MMA_THREADS, 0, st>>>(w, A, m, n, sp.ns > 1 ? part : c, sp.ns > 1 ? m : ldc, nrb, ncb, tiles,
                                                      sp.per, slice, sp.ns > 1 ? Epi{} : ep);
     return sp.ns > 1 ? launch_split_reduce(part, sp.ns, slice, m, n, c, ldc, st, ep) : hipGetLastError();
@@ -1250,7 +1243,10 @@ size_t gemm_mma_split_floats(int dt, int k, int m, int n) {
     if (dt != Q4_K && dt != Q5_K && dt != Q6_K && dt != MXFP4 && dt != Q4_0 && dt != Q8_0 && dt != NVFP4 && dt != Q1_0)
         return 0;
     const WidePlan wp = wide_of(dt, k, m, n);
-    const int ns = wp.wide ? wp.k.ns : split_plan(up_div(m, 32 * MMA_WAVES) * up_div(n, 64), up_div(k, 256)).ns;
+    const Split sp = dt == MXFP4 ? mx4_plan(m, k, n).k
+                     : wp.wide   ? wp.k
+                                 : split_plan(up_div(m, 32 * MMA_WAVES) * up_div(n, 64), up_div(k, 256));
+    const int ns = sp.ns;
     return ns > 1 ? (size_t) ns * n * m : 0;
 }
 
@@ -1287,7 +1283,7 @@ hipError_t launch_gemm_mma_grouped(int dt, const WeightView& w, const GemmAct& A
     case Q8_0: return kq_go<Q8_0, 1, 2>(w, A, g.gm, A.NP, c, ldc, st, g);
     case Q6_K: return kq_go<Q6_K, 1, 2>(w, A, g.gm, A.NP, c, ldc, st, g);
     case MXFP4:   // cap64 slot blocks at the most: the real count is on the device
-        return launch_mx4_gemm(w, A, g.gm, A.NP, c, ldc, st, g, mx4_rt(g.gm, A.K, cap64), 1, 0, 0, 0, Epi{});
+        return launch_mx4_gemm(w, A, g.gm, A.NP, c, ldc, st, g, mx4_row_tiles(g.gm, A.K, cap64), 1, 0, 0, 0, Epi{});
     default: return hipErrorNotSupported;
     }
 }

@@ -82,4 +82,19 @@ inline WidePlan wide_plan(int dt, int k, int m, int n, int cus, size_t act_bytes
     return {wide < other, s};
 }
 
+// MXFP4 (mx4.hip): waves of 64 rows (256-row workgroups, k whole) once those give each CU one, or at k <= 4096, where a
+// whole k is short, once they give every third CU one; else waves of 32 rows with the K split of the other types.
+// 64 against 32 rows: 14336x4096 n = 320 55.7 / 67.2 us (280 workgroups), n = 512 72.8 / 80.1, n = 128 36.5 / 38.8 (112),
+// 5760x2880 n = 256 27.5 / 32.0 (92), n = 512 37.9 / 41.8; but 14336x4096 n = 64 34.4 / 24.7 (56), 4096x14336 n = 512 111 /
+// 84 (128). A whole k of 64-row waves split like the others measures as the 32-row waves do.
+inline int mx4_row_tiles(int m, int k, int ncb) { return m >= 512 && up_div(m, 256) * ncb >= (k <= 4096 ? 88 : 256) ? 2 : 1; }
+struct Mx4Plan {
+    int rt, tiles;   // row tiles per wave, workgroup tiles
+    Split k;
+};
+inline Mx4Plan mx4_plan(int m, int k, int n) {
+    const int ncb = up_div(n, 64), rt = mx4_row_tiles(m, k, ncb), tiles = up_div(m, 128 * rt) * ncb;
+    return {rt, tiles, rt == 1 ? split_plan(tiles, up_div(k, 256)) : Split{1, 0}};
+}
+
 }  // namespace jamhip

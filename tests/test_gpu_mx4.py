@@ -54,3 +54,24 @@ def test_mx4_exact_blocks(hip, oracle, monkeypatch, m, n, k, lo, hi, extreme):
     err = np.abs(c[:, :m].astype(np.float64) - ref)
     assert (err <= bound).all(), (m, n, k, float((err / bound).max()))
     assert (c[:, m:] == -7.0).all()
+
+
+def test_mx4_noalloc_takes_no_unused_scratch(hip, oracle):
+    """5760 tokens on waves of 64 rows, whose k is never split: 50 MB of activations, inside the static 64 MiB without the 24 MB
+    of partial sums that two K slices would add."""
+    import torch
+    from qxotic_amd.jam import JAM, Segment
+    m, n, k = 512, 5760, 4096
+    w = blocks(np.random.default_rng(5), m, k, 110, 126, False)
+    a = torch.from_numpy(oracle.normal(6, (n, k))).cuda()
+    c, ref = torch.zeros((n, m), device="cuda"), torch.ones((n, m), device="cuda")
+    assert hip.pin(Segment.of(w), JAM.MXFP4, k, m) == JAM.OK, hip.last_error()
+    try:
+        torch.cuda.synchronize()
+        assert hip.mm_device(Segment.of(w), JAM.MXFP4, k, a.data_ptr(), k, ref.data_ptr(), m, m, n, k) == JAM.OK
+        st = hip.mm_device_noalloc(Segment.of(w), JAM.MXFP4, k, a.data_ptr(), k, c.data_ptr(), m, m, n, k)
+        assert st == JAM.OK, hip.last_error()
+        hip.synchronize()
+        assert torch.equal(c, ref)
+    finally:
+        hip.evict(Segment.of(w))

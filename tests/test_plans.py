@@ -16,6 +16,7 @@ extern "C" void q_wide(int dt, int k, int m, int n, size_t act, int* o) {
     const WidePlan p = wide_plan(dt, k, m, n, 256, act);
     o[0] = p.wide, o[1] = p.k.ns, o[2] = p.k.per;
 }
+extern "C" void q_mx4(int m, int k, int n, int* o) { const Mx4Plan p = mx4_plan(m, k, n); o[0] = p.rt, o[1] = p.tiles, o[2] = p.k.ns, o[3] = p.k.per; }
 extern "C" void q_split(int total, int units, int* o) { const Split s = split_plan(total, units); o[0] = s.ns, o[1] = s.per; }
 extern "C" int q_tail(int total, int cus) { return tail_tiles(total, cus); }
 """
@@ -34,6 +35,9 @@ class Plans:
         np_, sums = (n + 63) // 64 * 64, 16 if dt == O.Q6_K else 8
         act = k * np_ * 2 + k // 32 * np_ * 4 + 2 * (k // 256 * np_ * sums * 2) + 4 * np_
         return self._get("q_wide", 3, dt, k, m, n, ctypes.c_size_t(act))
+
+    def mx4(self, m, k, n):
+        return self._get("q_mx4", 4, m, k, n)
 
     def split(self, total, units):
         return self._get("q_split", 2, total, units)
@@ -88,3 +92,18 @@ def test_wide_offsets_fit_32_bits(plans):
     most = max(n for n in (1 << 16, 1 << 20, (1 << 22) - 64, 1 << 22, (1 << 22) + 1, 5 << 20, 1 << 23, 1 << 24)
                if plans.wide(O.Q6_K, 256, 512, n)[0])
     assert 11 * 64 * ((most + 63) // 64 * 64) < 1 << 32
+
+
+def test_mx4_plan(plans):
+    """64-row waves never split k; 32-row waves split it like the other types, whole super-blocks that cover it."""
+    for m in (16, 511, 512, 2880, 14336):
+        for k in (32, 4096, 4128, 14336):
+            for n in (9, 64, 128, 512, 5120):
+                rt, tiles, ns, per = plans.mx4(m, k, n)
+                assert tiles == -(-m // (128 * rt)) * -(-n // 64)
+                nsb = -(-k // 256)
+                if rt == 2:
+                    assert (ns, per) == (1, 0)
+                else:
+                    assert [ns, per] == plans.split(tiles, nsb) and ((ns, per) == (1, 0) or per * (ns - 1) < nsb <= per * ns)
+    assert plans.mx4(14336, 4096, 512)[0] == 2 and plans.mx4(14336, 4096, 64)[0] == 1 and plans.mx4(4096, 14336, 512)[0] == 1
