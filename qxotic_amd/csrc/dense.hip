@@ -19,6 +19,7 @@
 //  * dense_mma_kernel (F16, and BF16 with rounded activations, past the GEMV): LDS-staged f16 / bf16 matrix cores.
 #include "common.h"
 #include "launch.h"
+#include "plan.h"
 
 #include <type_traits>
 
@@ -850,24 +851,12 @@ int dense_mma_planes(int dt, int n, int k) {
     return dt == F16 ? 2 : 1;
 }
 
-// K slices for a grid of `total` workgroups: about two workgroups per CU (the quantized GEMM's rule).
-static void dense_split(int total, int nstk, int* ns, int* st_per) {
-    int want = total >= 384 ? 1 : (512 + total - 1) / total;
-    want = want < nstk ? want : nstk;
-    *st_per = want > 1 ? (nstk + want - 1) / want : 0;
-    *ns = want > 1 ? (nstk + *st_per - 1) / *st_per : 1;
-}
-
-// Workgroups (K slices included) from which dense_big_kernel, one per CU, beats the 128 x 64 one: 128 of them: F16 4096x14336
-// n = 512 190 against 252 us, 4096x4096 n = 256 44.5 / 51; 56 x 5 (14336x4096 n = 128) 64 / 99.
-// Not with up to 64 tokens, where half of its tile is padding: BF16 512x14336 n = 2 43.4 against 51.1 us, 1000x8192 n = 16
-// 29.0 / 33.1, F16 8000x1024 n = 12 15.1 / 17.2.
-constexpr int DBG_MIN_TILES = 128;
+// K slices, the quantized GEMM's rule over stages of 64
+static Split dense_split(int m, int n, int k) { return split_plan(up_div(m, 128) * (dense_np(n) / 64), dense_kp(k) / DMM_STAGE); }
 
 size_t dense_mma_split_floats(int dt, int k, int m, int n) {
     if (!dense_mma_planes(dt, n, k)) return 0;
-    int ns, st_per;
-    dense_split(((m + 127) / 128) * (dense_np(n) / 64), dense_kp(k) / DMM_STAGE, &ns, &st_per);
+    const int ns = dense_split(m, n, k).ns;
     return ns > 1 ? (size_t) ns * n * m : 0;
 }
 
@@ -886,21 +875,22 @@ hipError_t launch_dense_mma(int dt, const WeightView& w, const float* a, int lda
         dense_prep_few_kernel<<<n, 256, 0, st>>>(a, lda, n, k, Kp, NP, pl == 2, xh, pl == 2 ? xl : xh, es);
     else
         dense_prep_kernel<<<dim3((unsigned) ptiles, (unsigned) (pwant < pmax ? pwant : pmax)), 512, 0, st>>>(a, lda, n, k, Kp, NP, pl == 2, xh, pl == 2 ? xl : xh, es);
-    int nrb = (m + 127) / 128, ncb = NP / 64, ns, st_per;
-    dense_split(nrb * ncb, Kp / DMM_STAGE, &ns, &st_per);
+    const Split sp = dense_split(m, n, k);
+    const int ns = sp.ns, st_per = sp.per;
     if (ns > 1 && part == nullptr) return hipErrorInvalidValue;
     float* out = ns > 1 ? part : c;
     const int ldo = ns > 1 ? m : ldc;
     const int64_t slice = (int64_t) n * m;
     const Epi epo = ns > 1 ? Epi{} : ep;
-    const int brb = (m + 255) / 256, bcb = (NP + 127) / 128;
-    if (NP > 64 && brb * bcb * ns >= DBG_MIN_TILES) {   // the same K slices
+    if (dense_big(dt, Kp / DMM_STAGE, m, n, sp, device_cus())) {
+        const int brb = (m + 255) / 256, bcb = (NP + 127) / 128;
         const dim3 grid((unsigned) tile_grid(false, brb * bcb), (unsigned) ns);
         if (pl == 2)
             dense_big_kernel<true><<<grid, 512, 0, st>>>(w, xh, xl, es, NP, Kp, k, m, n, out, ldo, brb, bcb, st_per, slice, epo);
         else
             dense_big_kernel<false><<<grid, 512, 0, st>>>(w, xh, xh, es, NP, Kp, k, m, n, out, ldo, brb, bcb, st_per, slice, epo);
     } else {
+        const int nrb = (m + 127) / 128, ncb = NP / 64;
         const dim3 grid((unsigned) tile_grid(false, nrb * ncb), (unsigned) ns);
         const size_t lds = 2 * (size_t) (4 * 4096 + pl * 8192);
         if (pl == 2)

@@ -97,4 +97,24 @@ inline Mx4Plan mx4_plan(int m, int k, int n) {
     return {rt, tiles, rt == 1 ? split_plan(tiles, up_div(k, 256)) : Split{1, 0}};
 }
 
+// The staged dense GEMMs (F16, and BF16 with rounded activations): dense_mma_kernel's 128 x 64 tiles, two workgroups per CU, or
+// dense_big_kernel's 256 x 128, one per CU, over the same K slices of `units` stages of 64. As for the K-quants, what the
+// fullest CU computes decides, in stages of a 128 x 64 tile, of which a CU overlaps two and which ends with 2 more (BF16 0.5): a
+// stage of a big tile takes 1.7 of them (1.3), its start and end, which nothing on its CU overlaps, 5 (4), and the call 5 (8).
+// Both kernels over the same prep in 320 F16 and 320 BF16 calls (34 shapes from 32x2880 to 60000x256, 65 to 1024 tokens),
+// in us, big first:
+//   F16 14336x4096 n = 512 121 / 229, n = 65 (3 slices) 53 / 85; 6144x4096 n = 80 31 / 41; 8192x4096 n = 1024 132 / 229;
+//   4096x14336 n = 129 91 / 142; but 257x4096 n = 128 (22 slices of 3 stages) 76 / 42, 256x4096 n = 512 37 / 27,
+//   1000x1024 n = 256 26 / 24, 4096x128 n = 512 25 / 23, 32x2880 n = 512 36 / 27; BF16 256x4096 n = 512 33 / 24, 18910x192
+//   n = 881 61 / 52.
+// One call that the rule gives to the big tiles is 2% slower for it (F16 4096x4096 n = 512 62.4 / 61.1), the others no more than
+// 1.3%. Up to 64 tokens half of a big tile is padding and nothing is gained (F16 14336x4096 n = 16 58.2 / 58.2, BF16 n = 64
+// 55.4 / 53.1).
+inline bool dense_big(int dt, int units, int m, int n, Split s, int cus) {
+    if (n <= 64) return false;
+    const int per = s.ns > 1 ? s.per : units, big = cu_half_tiles(up_div(m, 256) * up_div(n, 128), s.ns, cus, false) / 2,
+              other = cu_half_tiles(up_div(m, 128) * up_div(n, 64), s.ns, cus, false) / 2;
+    return dt == F16 ? big * (1.7 * per + 5) + 5 < other * (per + 2.0) : big * (1.3 * per + 4) + 8 < other * (per + 0.5);
+}
+
 }  // namespace jamhip

@@ -17,6 +17,10 @@ extern "C" void q_wide(int dt, int k, int m, int n, size_t act, int* o) {
     o[0] = p.wide, o[1] = p.k.ns, o[2] = p.k.per;
 }
 extern "C" void q_mx4(int m, int k, int n, int* o) { const Mx4Plan p = mx4_plan(m, k, n); o[0] = p.rt, o[1] = p.tiles, o[2] = p.k.ns, o[3] = p.k.per; }
+extern "C" int q_big(int dt, int m, int k, int n) {
+    const int units = up_div(k, 64);
+    return dense_big(dt, units, m, n, split_plan(up_div(m, 128) * up_div(n, 64), units), 256);
+}
 extern "C" void q_split(int total, int units, int* o) { const Split s = split_plan(total, units); o[0] = s.ns, o[1] = s.per; }
 extern "C" int q_tail(int total, int cus) { return tail_tiles(total, cus); }
 """
@@ -107,3 +111,22 @@ def test_mx4_plan(plans):
                 else:
                     assert [ns, per] == plans.split(tiles, nsb) and ((ns, per) == (1, 0) or per * (ns - 1) < nsb <= per * ns)
     assert plans.mx4(14336, 4096, 512)[0] == 2 and plans.mx4(14336, 4096, 64)[0] == 1 and plans.mx4(4096, 14336, 512)[0] == 1
+
+
+# (type, m, k, n, the 256 x 128 tiles are faster), both measured over the same prep and K slices; 4% or more apart
+BIG = [(O.F16, 14336, 4096, 512, True), (O.F16, 14336, 4096, 65, True), (O.F16, 6144, 4096, 80, True), (O.F16, 4096, 14336, 129, True),
+       (O.F16, 8192, 4096, 1024, True), (O.F16, 257, 4096, 128, False), (O.F16, 256, 4096, 512, False), (O.F16, 1000, 1024, 256, False),
+       (O.F16, 4096, 128, 512, False), (O.F16, 32, 2880, 512, False), (O.F16, 128, 4096, 256, False), (O.F16, 512, 8192, 128, False),
+       (O.BF16, 14336, 4096, 512, True), (O.BF16, 14336, 4096, 128, True), (O.BF16, 2048, 14336, 192, True),
+       (O.BF16, 256, 4096, 512, False), (O.BF16, 257, 4096, 96, False), (O.BF16, 32, 2880, 512, False), (O.BF16, 512, 8192, 384, False),
+       (O.BF16, 18910, 192, 881, False), (O.F16, 50000, 768, 512, True)]
+
+
+@pytest.mark.parametrize("dt,m,k,n,big", BIG)
+def test_big_dense_tiles_where_they_are_faster(plans, dt, m, k, n, big):
+    assert bool(plans.lib.q_big(dt, m, k, n)) == big
+
+
+def test_big_dense_tiles_never_for_few_tokens(plans):
+    assert not any(plans.lib.q_big(dt, m, k, n) for dt in (O.F16, O.BF16) for m in (32, 4096, 200000) for k in (64, 14336)
+                   for n in (2, 9, 64))
