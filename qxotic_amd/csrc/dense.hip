@@ -386,6 +386,7 @@ __global__ void __launch_bounds__(512) dense_prep_kernel(const float* __restrict
     __shared__ float sdown[8];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int t0 = 8 * blockIdx.x;
+    if (t0 >= n) return;   // the whole workgroup: the grid is padded (dense_prep_grid)
     if (hl && t0 + wave < n) {   // a non-finite largest |x| leaves the scale at 1 (the outputs go non-finite)
         const float* x = a + (int64_t) (t0 + wave) * lda;
         float mx = 0.0f;
@@ -869,12 +870,11 @@ hipError_t launch_dense_mma(int dt, const WeightView& w, const float* a, int lda
     uint16_t* xh = (uint16_t*) scratch;
     uint16_t* xl = (uint16_t*) ((uint8_t*) scratch + plane);
     float* es = (float*) ((uint8_t*) scratch + pl * plane);
-    // about two workgroups per CU, each with at least one pass of 64 runs
-    const int ptiles = (n + 7) / 8, pmax = (Kp / 8 + 63) / 64, pwant = (512 + ptiles - 1) / ptiles;
+    const PrepGrid pg = dense_prep_grid(n, Kp);
     if (n <= 64)
         dense_prep_few_kernel<<<n, 256, 0, st>>>(a, lda, n, k, Kp, NP, pl == 2, xh, pl == 2 ? xl : xh, es);
     else
-        dense_prep_kernel<<<dim3((unsigned) ptiles, (unsigned) (pwant < pmax ? pwant : pmax)), 512, 0, st>>>(a, lda, n, k, Kp, NP, pl == 2, xh, pl == 2 ? xl : xh, es);
+        dense_prep_kernel<<<dim3((unsigned) pg.x, (unsigned) pg.y), 512, 0, st>>>(a, lda, n, k, Kp, NP, pl == 2, xh, pl == 2 ? xl : xh, es);
     const Split sp = dense_split(m, n, k);
     const int ns = sp.ns, st_per = sp.per;
     if (ns > 1 && part == nullptr) return hipErrorInvalidValue;

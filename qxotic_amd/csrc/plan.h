@@ -117,4 +117,16 @@ inline bool dense_big(int dt, int units, int m, int n, Split s, int cus) {
     return dt == F16 ? big * (1.7 * per + 5) + 5 < other * (per + 2.0) : big * (1.3 * per + 4) + 8 < other * (per + 0.5);
 }
 
+// dense_prep_kernel's grid: x over groups of 8 tokens, y over runs of their rows (of Kp elements), about two workgroups per CU,
+// each with at least one pass of 64 runs. Workgroups go to the XCDs in turn, so past 8 groups x is a multiple of 8: a group's
+// runs, each of which looks through the whole rows for the largest |x|, then share one L2. With 59 groups their rows went
+// through all eight (F16 k = 14336 n = 469 72 -> 49 us with the product, n = 1000 85 -> 63; k = 4096 n = 136 30.3 -> 28.4).
+struct PrepGrid {
+    int x, y;
+};
+inline PrepGrid dense_prep_grid(int n, int Kp) {
+    const int groups = up_div(n, 8), most = up_div(Kp / 8, 64), want = up_div(512, groups);
+    return {groups > 8 ? up_div(groups, 8) * 8 : groups, want < most ? want : most};
+}
+
 }  // namespace jamhip

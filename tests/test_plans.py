@@ -21,6 +21,7 @@ extern "C" int q_big(int dt, int m, int k, int n) {
     const int units = up_div(k, 64);
     return dense_big(dt, units, m, n, split_plan(up_div(m, 128) * up_div(n, 64), units), 256);
 }
+extern "C" void q_prep_grid(int n, int Kp, int* o) { const PrepGrid g = dense_prep_grid(n, Kp); o[0] = g.x, o[1] = g.y; }
 extern "C" void q_split(int total, int units, int* o) { const Split s = split_plan(total, units); o[0] = s.ns, o[1] = s.per; }
 extern "C" int q_tail(int total, int cus) { return tail_tiles(total, cus); }
 """
@@ -42,6 +43,9 @@ class Plans:
 
     def mx4(self, m, k, n):
         return self._get("q_mx4", 4, m, k, n)
+
+    def prep_grid(self, n, kp):
+        return self._get("q_prep_grid", 2, n, kp)
 
     def split(self, total, units):
         return self._get("q_split", 2, total, units)
@@ -130,3 +134,14 @@ def test_big_dense_tiles_where_they_are_faster(plans, dt, m, k, n, big):
 def test_big_dense_tiles_never_for_few_tokens(plans):
     assert not any(plans.lib.q_big(dt, m, k, n) for dt in (O.F16, O.BF16) for m in (32, 4096, 200000) for k in (64, 14336)
                    for n in (2, 9, 64))
+
+
+def test_dense_prep_grid(plans):
+    """Every group of 8 tokens and every run of 8 elements has a workgroup, and the workgroups of a group (x, x + gridDim.x, ... in
+    launch order, dealt to the 8 XCDs in turn) meet on one XCD once there are groups for all."""
+    for n in (2, 9, 64, 65, 72, 136, 197, 300, 469, 512, 1000, 4150):
+        for kp in (64, 512, 2048, 2880, 14336):
+            x, y = plans.prep_grid(n, kp)
+            groups = -(-n // 8)
+            assert groups <= x < groups + 8 and 1 <= y <= max(1, -(-kp // 512))
+            assert groups <= 8 or len({(x * i) % 8 for i in range(y)}) == 1
