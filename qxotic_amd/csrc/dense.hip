@@ -454,9 +454,7 @@ __global__ void __launch_bounds__(512) dense_prep_kernel(const float* __restrict
     }
 }
 
-// Up to 64 tokens: a workgroup per token, which reads its row in whole lines; there are too few tokens for the form above to
-// fill the CUs, and its scattered reads show: F16 512x1024 n = 40 14.3 against 15.0 us, 1000x1024 n = 9 12.4 / 12.9, BF16
-// 11.5 / 11.9 (F16 of 8 to 16 tokens at k = 4096, whose largest |x| takes one wave longer here: 18.3 / 17.2).
+// Short rows of few tokens (dense_prep_few): a workgroup per token, which reads its row in whole lines.
 __global__ void __launch_bounds__(256) dense_prep_few_kernel(const float* __restrict__ a, int lda, int n, int k, int Kp,
                                                          int NP, int hl, uint16_t* __restrict__ hi,
                                                          uint16_t* __restrict__ lo, float* __restrict__ es) {
@@ -871,7 +869,7 @@ hipError_t launch_dense_mma(int dt, const WeightView& w, const float* a, int lda
     uint16_t* xl = (uint16_t*) ((uint8_t*) scratch + plane);
     float* es = (float*) ((uint8_t*) scratch + pl * plane);
     const PrepGrid pg = dense_prep_grid(n, Kp);
-    if (n <= 64)
+    if (dense_prep_few(dt, k, n))
         dense_prep_few_kernel<<<n, 256, 0, st>>>(a, lda, n, k, Kp, NP, pl == 2, xh, pl == 2 ? xl : xh, es);
     else
         dense_prep_kernel<<<dim3((unsigned) pg.x, (unsigned) pg.y), 512, 0, st>>>(a, lda, n, k, Kp, NP, pl == 2, xh, pl == 2 ? xl : xh, es);

@@ -129,4 +129,13 @@ inline PrepGrid dense_prep_grid(int n, int Kp) {
     return {groups > 8 ? up_div(groups, 8) * 8 : groups, want < most ? want : most};
 }
 
+// Which form of the dense activation prep: a workgroup per token (true), or 8 tokens per workgroup, the row cut into runs. The
+// first reads its row in whole lines and finds its largest |x| (F16) in one pass; the second fills the CUs once rows are long
+// or tokens many. By row length and tokens, measured apart from the tile form (us with the product, first form against second):
+// F16 k = 512 n = 271 17.5 / 18.0; k = 1024 n = 9 12.6 / 13.1, n = 128 18.8 / 19.3, n = 512 23.4 / 23.1; k = 2000 n = 9 16.4 /
+// 17.0, n = 300 21.9 / 21.0; k = 2048 n = 256 21.8 / 21.1; k = 4096 n = 9 25.4 / 24.5, n = 64 33.5 / 31.2; k = 14336 n = 9
+// 86 / 73; BF16 (no largest |x|) k = 2000 n = 64 18.2 / 18.3, n = 512 19.5 / 18.5; k = 2048 n = 9 14.9 / 15.3; k = 4096 n = 64
+// 29.2 / 28.6; k = 14336 n = 64 76 / 73.
+inline bool dense_prep_few(int dt, int k, int n) { return n <= (k <= 1024 ? 320 : 256) && k <= (dt == F16 ? 2047 : 2048); }
+
 }  // namespace jamhip

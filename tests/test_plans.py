@@ -22,6 +22,7 @@ extern "C" int q_big(int dt, int m, int k, int n) {
     return dense_big(dt, units, m, n, split_plan(up_div(m, 128) * up_div(n, 64), units), 256);
 }
 extern "C" void q_prep_grid(int n, int Kp, int* o) { const PrepGrid g = dense_prep_grid(n, Kp); o[0] = g.x, o[1] = g.y; }
+extern "C" int q_few(int dt, int k, int n) { return dense_prep_few(dt, k, n); }
 extern "C" void q_split(int total, int units, int* o) { const Split s = split_plan(total, units); o[0] = s.ns, o[1] = s.per; }
 extern "C" int q_tail(int total, int cus) { return tail_tiles(total, cus); }
 """
@@ -145,3 +146,11 @@ def test_dense_prep_grid(plans):
             groups = -(-n // 8)
             assert groups <= x < groups + 8 and 1 <= y <= max(1, -(-kp // 512))
             assert groups <= 8 or len({(x * i) % 8 for i in range(y)}) == 1
+
+
+@pytest.mark.parametrize("dt,k,n,few", [(O.F16, 4096, 9, False), (O.F16, 4096, 64, False), (O.F16, 14336, 9, False), (O.F16, 1024, 9, True),
+                                        (O.F16, 1024, 128, True), (O.F16, 512, 192, True), (O.F16, 2000, 64, True), (O.F16, 2048, 256, False),
+                                        (O.F16, 1024, 1024, False), (O.BF16, 1024, 128, True), (O.BF16, 4096, 64, False),
+                                        (O.BF16, 14336, 9, False), (O.BF16, 2048, 1024, False)])
+def test_dense_prep_form_that_is_faster(plans, dt, k, n, few):
+    assert bool(plans.lib.q_few(dt, k, n)) == few
