@@ -264,7 +264,7 @@ constexpr int DT_WAVES = 8;
 template <int DT, int T>
 __global__ void __launch_bounds__(64 * DT_WAVES) dense_tile_kernel(WeightView w, const float* __restrict__ a, int lda,
                                                                    int k, int m, int n, float* __restrict__ c, int ldc,
-                                                                   int nt, int vec, Epi ep) {
+                                                                   int nt, Epi ep) {
     constexpr int Q = 64 / T, RUN = 16 * Q, E = T * T / 64, LD = T + 4;
     constexpr int ES = block_bytes(DT);
     static_assert(DT == F32 || DT == BF16, "F16 takes the staged GEMM");
@@ -281,24 +281,27 @@ __global__ void __launch_bounds__(64 * DT_WAVES) dense_tile_kernel(WeightView w,
     // Piece i of a run is 4·Q consecutive k of a row, 4 per lane, so a load instruction reads 16·Q (F32) contiguous bytes
     // of T rows. A run never crosses a row's 256-byte pitch (RUN·ES divides it): weight loads past k stay in the row.
     typedef uint32_t piece __attribute__((ext_vector_type(ES)));   // 4 weights
-    auto load = [&](piece (&wv)[4], float4 (&xv)[4], int it) {
+    // Activation rows start at any 4-byte address (row strides are the caller's): gfx950 loads 16 bytes from there in one
+    // instruction, where element-wise loads made odd strides slow (F32 41478x634 n = 190 314 -> 178 us, 42665x1090 n = 255 734 -> 382).
+    typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+    auto load = [&](piece (&wv)[4], f32x4u (&xv)[4], int it) {
         const int e0 = it * RUN + 4 * q;
 #pragma unroll
         for (int i = 0; i < 4; i++) wv[i] = *reinterpret_cast<const piece*>(wp + (int64_t) (e0 + 4 * Q * i) * ES);
-        if (vec && (it + 1) * RUN <= k) {   // wave-uniform
+        if ((it + 1) * RUN <= k) {   // wave-uniform
 #pragma unroll
-            for (int i = 0; i < 4; i++) xv[i] = *reinterpret_cast<const float4*>(ap + e0 + 4 * Q * i);
+            for (int i = 0; i < 4; i++) xv[i] = *reinterpret_cast<const f32x4u*>(ap + e0 + 4 * Q * i);
         } else {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int e = e0 + 4 * Q * i;
-                xv[i] = make_float4(e < k ? ap[e] : 0.0f, e + 1 < k ? ap[e + 1] : 0.0f, e + 2 < k ? ap[e + 2] : 0.0f,
-                                    e + 3 < k ? ap[e + 3] : 0.0f);
+                xv[i] = f32x4u{e < k ? ap[e] : 0.0f, e + 1 < k ? ap[e + 1] : 0.0f, e + 2 < k ? ap[e + 2] : 0.0f,
+                               e + 3 < k ? ap[e + 3] : 0.0f};
             }
         }
     };
     accv acc[2] = {accv{}, accv{}};
-    auto mul = [&](const piece (&wv)[4], const float4 (&xv)[4], int it) {
+    auto mul = [&](const piece (&wv)[4], const f32x4u (&xv)[4], int it) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             float f[4];
@@ -314,19 +317,18 @@ __global__ void __launch_bounds__(64 * DT_WAVES) dense_tile_kernel(WeightView w,
 #pragma unroll
                 for (int u = 0; u < 4; u++) f[u] = it * RUN + 4 * q + 4 * Q * i + u < k ? f[u] : 0.0f;
             }
-            const float x[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 if constexpr (T == 16)
-                    acc[u & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[u], x[u], acc[u & 1], 0, 0, 0);
+                    acc[u & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[u], xv[i][u], acc[u & 1], 0, 0, 0);
                 else
-                    acc[u & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(f[u], x[u], acc[u & 1], 0, 0, 0);
+                    acc[u & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(f[u], xv[i][u], acc[u & 1], 0, 0, 0);
             }
         }
     };
     for (int it = wave; it < runs; it += DT_WAVES) {
         piece wv[4];
-        float4 xv[4];
+        f32x4u xv[4];
         load(wv, xv, it);
         mul(wv, xv, it);
     }
@@ -822,16 +824,15 @@ static hipError_t dense_go(const WeightView& w, const float* a, int lda, int k, 
     }
     // F16 and bf16-rounded BF16 calls of 2 or more tokens past the GEMV took the staged GEMM (dense_mma_planes)
     if constexpr (DT != F16) {
-        const int vec = lda % 4 == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0;
         const int64_t nt32 = (n + 31) / 32, tiles32 = (int64_t) ((m + 31) / 32) * nt32;
         const int64_t nt16 = (n + 15) / 16, tiles16 = (int64_t) ((m + 15) / 16) * nt16;
         if (tiles32 > 0x7fffffff) return hipErrorInvalidValue;
         if (tiles32 >= DENSE_TILE32_MIN)
             dense_tile_kernel<DT, 32><<<(unsigned) tiles32, 64 * DT_WAVES, 0, st>>>(w, a, lda, k, m, n, c, ldc, (int) nt32,
-                                                                                    vec, ep);
+                                                                                    ep);
         else
             dense_tile_kernel<DT, 16><<<(unsigned) tiles16, 64 * DT_WAVES, 0, st>>>(w, a, lda, k, m, n, c, ldc, (int) nt16,
-                                                                                    vec, ep);
+                                                                                    ep);
         return hipGetLastError();
     }
     return hipErrorInvalidValue;
