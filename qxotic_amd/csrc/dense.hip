@@ -256,9 +256,6 @@ __global__ void __launch_bounds__(64 * DG_WAVES) dense_gemv2_kernel(WeightView w
 // more than twice as fast where the tiles fill the chip (F32 4096x4096 n = 512: 556 -> 255 us; 2048x2880 n = 512:
 // 391 -> 95). Two or three runs in flight per wave instead of one lose 5 to 30%: the registers cost more waves than the
 // distance hides. The waves' sums meet in LDS in a fixed order.
-// 32 x 32 tiles halve the bytes read per product and take over once they give most CUs one (F32 512x2880 n = 512, 256 such
-// tiles: 25 against 50.8 us; 1024x2880 n = 128, 128 tiles, stays with 16 x 16: 24.4 us).
-constexpr int64_t DENSE_TILE32_MIN = 192;
 constexpr int DT_WAVES = 8;
 
 template <int DT, int T>
@@ -826,8 +823,8 @@ static hipError_t dense_go(const WeightView& w, const float* a, int lda, int k, 
     if constexpr (DT != F16) {
         const int64_t nt32 = (n + 31) / 32, tiles32 = (int64_t) ((m + 31) / 32) * nt32;
         const int64_t nt16 = (n + 15) / 16, tiles16 = (int64_t) ((m + 15) / 16) * nt16;
-        if (tiles32 > 0x7fffffff) return hipErrorInvalidValue;
-        if (tiles32 >= DENSE_TILE32_MIN)
+        if (tiles32 > 0x7fffffff) return hipErrorInvalidValue;   // (16 x 16 tiles: n <= 16 or few)
+        if (dense_tile32(m, n))
             dense_tile_kernel<DT, 32><<<(unsigned) tiles32, 64 * DT_WAVES, 0, st>>>(w, a, lda, k, m, n, c, ldc, (int) nt32,
                                                                                     ep);
         else

@@ -138,4 +138,10 @@ inline PrepGrid dense_prep_grid(int n, int Kp) {
 // 29.2 / 28.6; k = 14336 n = 64 76 / 73.
 inline bool dense_prep_few(int dt, int k, int n) { return n <= (k <= 1024 ? 320 : 256) && k <= (dt == F16 ? 2047 : 2048); }
 
+// dense_tile_kernel's tile: 32 x 32 (true) halves the bytes read per product and takes over once such tiles give most CUs one,
+// but up to 16 tokens half of it is padding. 16 x 16 against 32 x 32, us: F32 512x2880 n = 512 (256 tiles of 32) 41.4 / 24.6,
+// 2048x4096 n = 96 (192) 44.5 / 32.7; 256x4096 n = 512 (128) 30.6 / 32.1, 2048x4096 n = 64 (128) 30.8 / 32.2; 14336x4096
+// n = 5 49 / 71, n = 16 62 / 71, n = 17 (448) 101 / 71, 32000x2048 n = 9 54 / 68.
+inline bool dense_tile32(int m, int n) { return n > 16 && (int64_t) up_div(m, 32) * up_div(n, 32) >= 192; }
+
 }  // namespace jamhip

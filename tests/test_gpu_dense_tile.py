@@ -12,7 +12,8 @@ from oracle import oracle as O
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(1, 9, 1), (8, 512, 544), (15, 16, 63), (16, 17, 64), (17, 31, 65), (32, 512, 2880), (33, 33, 511), (64, 300, 1000),
-          (600, 40, 96), (256, 1, 2880), (257, 2, 100), (3, 4, 1024), (32, 8, 31), (31, 5, 2881), (2048, 64, 33)]
+          (600, 40, 96), (256, 1, 2880), (257, 2, 100), (3, 4, 1024), (32, 8, 31), (31, 5, 2881), (2048, 64, 33),
+          (6200, 16, 70), (6200, 17, 70), (4100, 5, 4099)]
 
 
 @pytest.mark.parametrize("m,n,k", SHAPES)

@@ -23,6 +23,7 @@ extern "C" int q_big(int dt, int m, int k, int n) {
 }
 extern "C" void q_prep_grid(int n, int Kp, int* o) { const PrepGrid g = dense_prep_grid(n, Kp); o[0] = g.x, o[1] = g.y; }
 extern "C" int q_few(int dt, int k, int n) { return dense_prep_few(dt, k, n); }
+extern "C" int q_tile32(int m, int n) { return dense_tile32(m, n); }
 extern "C" void q_split(int total, int units, int* o) { const Split s = split_plan(total, units); o[0] = s.ns, o[1] = s.per; }
 extern "C" int q_tail(int total, int cus) { return tail_tiles(total, cus); }
 """
@@ -154,3 +155,9 @@ def test_dense_prep_grid(plans):
                                         (O.BF16, 14336, 9, False), (O.BF16, 2048, 1024, False)])
 def test_dense_prep_form_that_is_faster(plans, dt, k, n, few):
     assert bool(plans.lib.q_few(dt, k, n)) == few
+
+
+@pytest.mark.parametrize("m,n,big", [(14336, 5, False), (14336, 16, False), (32000, 9, False), (14336, 17, True), (512, 512, True),
+                                     (2048, 96, True), (2048, 64, False), (256, 512, False), (32, 512, False)])
+def test_f32_tile_that_is_faster(plans, m, n, big):
+    assert bool(plans.lib.q_tile32(m, n)) == big
