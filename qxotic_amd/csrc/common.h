@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "dtype.h"
+#include "plan.h"
 
 namespace jamhip {
 
@@ -54,11 +55,10 @@ __host__ __device__ constexpr int64_t groups_of(int dt, int64_t blocks) {
 // rows held by a device copy of m rows (whole 32-row tiles)
 __host__ __device__ constexpr int64_t tiled_rows(int64_t m) { return (m + ROW_TILE - 1) / ROW_TILE * ROW_TILE; }
 
-// Dense weights are kept row-major on the device, each row padded with zeros to an odd multiple of 256 bytes (so every row
-// starts 16-byte aligned for vector loads, the padding reads as zeros, and rows of a power-of-two length do not all start
-// on one memory channel: F16 4096x4096 n = 1 10.4 -> 9.4 us, 14336x4096 23.7 -> 22.8); WeightView::G then holds the
-// pitch in bytes. The sizes of a device copy of `rows` rows of `ldw` elements, for any weight type:
-__host__ __device__ constexpr int64_t dense_pitch(int dt, int64_t ldw) { return ((ldw * block_bytes(dt) + 255) / 256 | 1) * 256; }
+// Dense weights are kept row-major on the device, each row padded with zeros to dense_row_pitch (so every row starts 16-byte
+// aligned and the padding reads as zeros); WeightView::G then holds the pitch in bytes. The sizes of a device copy of
+// `rows` rows of `ldw` elements, for any weight type:
+__host__ __device__ constexpr int64_t dense_pitch(int dt, int64_t ldw) { return dense_row_pitch(ldw * block_bytes(dt)); }
 // WeightView::G of such a copy: groups per row (quantized) or the pitch (dense)
 __host__ __device__ constexpr int64_t view_G(int dt, int64_t ldw) {
     return is_dense(dt) ? dense_pitch(dt, ldw) : groups_of(dt, ldw / block_elems(dt));

@@ -7,8 +7,8 @@
 // and f32 x f32 products are formed exactly by the FMA / the matrix cores); only the f32 summation order
 // differs from jam's.
 //
-// Layout. A device copy keeps the rows row-major, each padded with zeros to a pitch of an odd multiple of 256 bytes (WeightView::G),
-// so every row starts 16-byte aligned and a 16-byte load never crosses into the next row.
+// Layout. A device copy keeps the rows row-major, each padded with zeros to a pitch of whole 256 bytes (dense_row_pitch,
+// WeightView::G), so every row starts 16-byte aligned and a 16-byte load never crosses into the next row.
 //
 // Kernels.
 //  * dense_gemv2_kernel (n <= 8 while the token tile's activations fit 64 KB of LDS; HBM-bound): activations
@@ -19,7 +19,6 @@
 //  * dense_mma_kernel (F16, and BF16 with rounded activations, past the GEMV): LDS-staged f16 / bf16 matrix cores.
 #include "common.h"
 #include "launch.h"
-#include "plan.h"
 
 #include <type_traits>
 

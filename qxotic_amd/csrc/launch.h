@@ -178,8 +178,8 @@ hipError_t launch_mx_gemm(int mode, const WeightView& w, const MxAct& A, int m, 
 hipError_t launch_mx_gemm_grouped(int mode, const WeightView& w, const MxAct& A, const Groups& g, int cap64, float* c,
                                   int ldc, hipStream_t st);
 
-// Dense weights (F32, F16, BF16; dense.hip): jam's dense paths, any n, any k (rows padded to a 256-byte pitch,
-// WeightView::G = the pitch).
+// Dense weights (F32, F16, BF16; dense.hip): jam's dense paths, any n, any k (rows padded to dense_row_pitch bytes,
+// WeightView::G).
 hipError_t launch_dense(int dt, const WeightView& w, const float* a, int lda, int k, int m, int n, float* c, int ldc,
                         hipStream_t st, const Epi& ep = Epi{});
 // From DENSE_MMA_MIN_N tokens (from 2 where the staged GEMV's activation tile would not fit LDS) F16, and BF16

@@ -30,7 +30,6 @@
 // weight tile is read from HBM into that XCD's L2 once.
 #include "common.h"
 #include "launch.h"
-#include "plan.h"
 
 #include <atomic>
 #include <type_traits>

@@ -11,6 +11,16 @@ namespace jamhip {
 
 inline int up_div(int a, int b) { return (a + b - 1) / b; }
 
+// Bytes from one row of a device copy of dense weights to the next. Rows start on 256 bytes, so 16-byte aligned for vector loads;
+// from 4096 bytes on the pitch is an odd multiple, so that rows of a power-of-two length do not all start on one memory
+// channel (one token, us, even against odd: F16 8192x2048 9.6 / 8.1, 32000x2048 26.8 / 23.5, 4096x4096 9.7 / 8.8, 14336x4096 23.5 /
+// 22.5, F32 32000x1024 26.1 / 22.0). Shorter rows share DRAM pages that the gap would break up (F16 32000x1024 n = 64 33.3 /
+// 37.7, 4096x256 n = 4 4.97 / 5.33), and would pay for it with up to half as much memory again; from there on it is 1/16 at most.
+constexpr int64_t dense_row_pitch(int64_t row_bytes) {
+    const int64_t units = (row_bytes + 255) / 256;
+    return (units >= 16 ? units | 1 : units) * 256;
+}
+
 // K slices of a matrix-core GEMM: ns of them, `per` K units each (0 when whole).
 struct Split {
     int ns, per;

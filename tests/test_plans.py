@@ -24,6 +24,7 @@ extern "C" int q_big(int dt, int m, int k, int n) {
 extern "C" void q_prep_grid(int n, int Kp, int* o) { const PrepGrid g = dense_prep_grid(n, Kp); o[0] = g.x, o[1] = g.y; }
 extern "C" int q_few(int dt, int k, int n) { return dense_prep_few(dt, k, n); }
 extern "C" int q_tile32(int m, int n) { return dense_tile32(m, n); }
+extern "C" long long q_pitch(long long bytes) { return dense_row_pitch(bytes); }
 extern "C" void q_split(int total, int units, int* o) { const Split s = split_plan(total, units); o[0] = s.ns, o[1] = s.per; }
 extern "C" int q_tail(int total, int cus) { return tail_tiles(total, cus); }
 """
@@ -32,6 +33,8 @@ extern "C" int q_tail(int total, int cus) { return tail_tiles(total, cus); }
 class Plans:
     def __init__(self, so):
         self.lib = ctypes.CDLL(str(so))
+
+        self.lib.q_pitch.restype, self.lib.q_pitch.argtypes = ctypes.c_longlong, [ctypes.c_longlong]
 
     def _get(self, name, size, *args):
         o = (ctypes.c_int * size)()
@@ -161,3 +164,15 @@ def test_dense_prep_form_that_is_faster(plans, dt, k, n, few):
                                      (2048, 96, True), (2048, 64, False), (256, 512, False), (32, 512, False)])
 def test_f32_tile_that_is_faster(plans, m, n, big):
     assert bool(plans.lib.q_tile32(m, n)) == big
+
+
+def test_dense_pitch(plans):
+    """A row fits and starts on 256 bytes; rows of 4096 bytes and more lie an odd number of 256 bytes apart, at most 1/16 further
+    than before that rule; shorter rows take no more memory than their 256-byte pieces."""
+    for b in [1, 2, 255, 256, 257, 512, 1024, 2048, 3841, 4095, 4096, 4097, 5760, 8192, 11520, 16384, 28672, 57344, 1 << 33]:
+        p, even = plans.lib.q_pitch(b), -(-b // 256) * 256
+        assert p >= b and p % 256 == 0
+        if even < 4096:
+            assert p == even
+        else:
+            assert p // 256 % 2 == 1 and p - even <= min(256, even // 16)
