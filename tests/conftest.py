@@ -49,6 +49,13 @@ def refjam_generic():
 
 
 @pytest.fixture(scope="session")
+def plans(tmp_path_factory):
+    """The rules that choose a kernel for a call (plans.Plans)."""
+    import plans as P
+    return P.build(tmp_path_factory.mktemp("plans"))
+
+
+@pytest.fixture(scope="session")
 def hip():
     from qxotic_amd.jam import HipJAM
     h = HipJAM()

@@ -19,15 +19,19 @@ def blocks(rng, m, k, lo, hi, extreme):
     return np.ascontiguousarray(b.reshape(m, -1))
 
 
+# 64-row waves over whole 64-token tiles, no half tile in the last round, several stages: the last one full and short
+FULL = [(1024, 4096, 288), (1024, 4090, 416)]
 # m in whole bands of 16: the last m % 16 rows of a call are a float dot on another kernel
 SHAPES = [(16, 9, 32), (32, 64, 96), (48, 65, 128), (96, 33, 160), (128, 40, 256), (160, 130, 288), (528, 77, 416), (544, 1920, 288),
-          (2880, 545, 96), (512, 31, 4096), (144, 8, 2880)]
+          (2880, 545, 96), (512, 31, 4096), (144, 8, 2880), *FULL]
 
 
 @pytest.mark.parametrize("m,n,k", SHAPES)
 @pytest.mark.parametrize("lo,hi,extreme", [(110, 126, False), (110, 126, True), (0, 14, False), (225, 238, False), (232, 254, False)])
-def test_mx4_exact_blocks(hip, oracle, monkeypatch, m, n, k, lo, hi, extreme):
+def test_mx4_exact_blocks(hip, oracle, plans, monkeypatch, m, n, k, lo, hi, extreme):
     from qxotic_amd.jam import JAM, Segment
+    rt, tiles, _, _ = plans.mx4(m, k, n)
+    assert (m, n, k) not in FULL or (rt, plans.lib.q_tail(tiles, 256)) == (2, 0)
     monkeypatch.setenv("JAM_HIP_MMA_MIN_N", "8")
     rng = np.random.default_rng(m + 31 * n + 977 * k + lo)
     w = blocks(rng, m, k, lo, hi, extreme)

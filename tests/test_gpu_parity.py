@@ -424,12 +424,15 @@ def test_prefill_ragged_shapes(hip, oracle, dt):
 
 
 @pytest.mark.parametrize("dt", [O.Q4_K, O.Q5_K, O.Q6_K, O.MXFP4, O.NVFP4, O.Q8_0, O.Q4_0, O.Q1_0])
-def test_prefill_tail_split_tiles(hip, oracle, dt):
+def test_prefill_tail_split_tiles(hip, oracle, plans, dt):
     """Grids whose last partial round of tiles runs as half tiles: 1024 rows x 65 slot blocks give 65 tiles per
-    XCD, one of them split into two 32-token workgroups. Every token's result equals that of the n = 4096 grid
-    (64 tiles per XCD, none split) bit for bit, and a row sample meets tier 1. n = 4150 leaves the second half
-    of the last slot block partly valid, n = 4110 leaves it empty."""
+    XCD (MXFP4, 256 rows a tile: 33), one of them split into two 32-token workgroups. Every token's result equals that
+    of the n = 4096 grid (64 and 32 tiles per XCD, none split) bit for bit, and a row sample meets tier 1. n = 4150
+    leaves the second half of the last slot block partly valid, n = 4110 leaves it empty."""
     m, k = 1024, 256
+    for n, tail in ((4096, 0), (4110, 1), (4150, 1)):
+        tiles = plans.mx4(m, k, n)[1] if dt == O.MXFP4 else m // 128 * -(-n // 64)
+        assert plans.lib.q_tail(tiles, 256) == tail and not plans.wide(dt, k, m, n)[0]
     w = oracle.quantize(dt, oracle.normal(0x7A11 ^ dt, (m, k), 0.0, 0.02))
     a = oracle.outliers(0x7A12, (4150, k))
     base = run_mm(hip, dt, w, np.ascontiguousarray(a[:4096]), m, 4096, k)
