@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "dtype.h"
 #include "plan.h"
 
@@ -28,7 +30,7 @@ __host__ __device__ constexpr bool is_dense(int dt) { return dt == F32 || dt == 
 //   Q6_K : NC 13 chunks 0-7 ql, 8-11 qh, 12 the 16 int8 scales | SB 2 : d fp16
 //   Q8_0 : NC 16 chunk c = half c&1 of block c>>1 (int8 q)     | SB 16: the 8 blocks' fp16 d
 //   Q4_0 : NC 8  chunk c = block c's 16 nibble bytes           | SB 16: the 8 blocks' fp16 d
-//   MXFP4: NC 8  chunk c = block c's 16 nibble bytes           | SB 16: the 8 blocks' e8m0, then their maximum
+//   MXFP4: NC 8  chunk c = block c's 16 nibble bytes           | SB 16: the 8 blocks' e8m0, 8 zero bytes
 //   Q5_K : NC 10 chunks 0-7 qs nibble bytes, 8-9 the qh bytes   | SB 16: d, dmin, 12 scale bytes
 //   NVFP4: NC 8  chunk 2j + h = half h of 64-block j's qs       | SB 16: the 4 blocks' 4 UE4M3 scales
 //   Q1_0 : NC 2  chunk j = 128-block j's 16 sign bytes          | SB 4 : the 2 blocks' fp16 d
@@ -161,6 +163,14 @@ struct ActQ {
 };
 
 #define JAMHIP_DEV __device__ __forceinline__
+
+// f(integral_constant I), ..., f(integral_constant N - 1)
+template <int I, int N, typename F> JAMHIP_DEV void unroll(const F& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        unroll<I + 1, N>(f);
+    }
+}
 
 JAMHIP_DEV float h2f(uint32_t bits16) { return (float) __builtin_bit_cast(_Float16, (uint16_t) bits16); }
 

@@ -871,11 +871,12 @@ __global__ void __launch_bounds__(MMA_THREADS, 2) kq_gemm_kernel(WeightView w, G
 
 // ------------------------------------------------------------------------------------------ wide kernel
 // The K-quants with more than 64 tokens: the same arithmetic, in waves of 32 rows x 128 tokens (a workgroup of 4 waves: 128
-// rows x 128 tokens), k in stages of 64 (two blocks). kq_gemm_kernel is bound by VALU issue (18 instructions per MFMA, a
-// third of them the weight decode): here a decoded fragment serves four token tiles instead of two (11 per MFMA), a stage's
-// copies go out at its start into a buffer of their own, fragments are read a step ahead, and products are issued between
-// the previous step's FMAs. Figures at wide_plan. Three stage buffers instead of two (Q4_K) measured slower (n = 512 116 us):
-// it is the copies' own issue and LDS traffic that cost, not their latency.
+// rows x 128 tokens), k in stages of 64 (two blocks). Against kq_gemm_kernel (18 VALU instructions per MFMA, a third of them the
+// weight decode) a decoded fragment serves four token tiles instead of two (12 per MFMA), a stage's copies go out at its
+// start into a buffer of their own, fragments are read a step ahead, and products are issued between the previous step's
+// FMAs. Neither pipe is full: 14336x4096 n = 512 has the VALU busy 46% of the time and the matrix cores 30% (Q6_K 53% and
+// 45%), and its waves wait for a stage's copies or the barrier 27% of theirs. Figures at wide_plan. Three stage buffers
+// instead of two (Q4_K) measured slower (n = 512 116 us).
 // Stage buffer: weight chunks [4 tiles][NCS][32 rows][16 B], row headers [4][32][HB], codes [2 blocks][2 K-steps][2 halves][128
 // tokens][16 B], block scales [2][128] f32; the buffer of a super-block's sums stage (the last for Q4_K / Q5_K, the first for
 // Q6_K) also holds their hi and lo planes [128 tokens][SW] f16.
@@ -887,13 +888,6 @@ template <int DT> struct WStage {
     static constexpr int H = 4 * NCS * 512, B = H + (128 * HB + 1023) / 1024 * 1024, DX = B + 16384, S = DX + 1024,
                          BYTES = S + 2 * 128 * SW * 2;
 };
-
-template <int I, int N, typename F> JAMHIP_DEV void unroll(const F& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        unroll<I + 1, N>(f);
-    }
-}
 
 template <int DT>
 __global__ void __launch_bounds__(MMA_THREADS, 2) kq_wide_kernel(WeightView w, GemmAct A, int m, int n,

@@ -9,14 +9,18 @@
 // result is 2^(e - 128)·Σ kv·q (kv jam's doubled codes, jam_mxfp4.h:14-24), which f32 holds exactly: |Σ kv·q| < 2^16.
 // Checked on the device against integer sums for random and extreme codes and every exponent up to 238 (subnormal
 // results included); the repack keeps tensors with larger ones, whose products could overflow, off this kernel. One f32
-// FMA per output then applies the block's activation scale, in groups of 8 blocks summed into the total as the f16 kernel
-// this replaces did: the results are bit-identical to it.
+// FMA per output then applies the block's activation scale, in groups of 8 blocks summed into the total. While every partial
+// sum is a normal, finite f32 the results are bit-identical to the f16 form this replaces, which summed a group in units of its
+// largest exponent and applied that once. Below, each block's FMA rounds at 2^-149 where that form rounded once a group;
+// and a block term past f32's largest is infinite before a later one could cancel it. jam applies every block's scale by
+// itself too, so its own sums round and overflow there.
 //
 // What bounds it. Nothing but that FMA is left per output and block (16 VALU instructions, 64 cycles of a SIMD, per
 // instruction of 33 cycles on the matrix cores, where the f16 form took two MFMAs and 8 conversions per 8 weights), so
 // the VALU issue rate is the ceiling, and LDS traffic is next: a wave of 32 x 64 outputs reads 32 cycles of fragments
 // per 32 cycles of its share of the FMAs. A wave therefore owns 64 rows x 64 tokens (RT = 2: the token fragments serve two
-// row tiles). With the prep, f16 kernel -> this one: 14336x4096 n = 512 103 -> 73 us, n = 2048 373 -> 240 us; the two
+// row tiles). It is not at that ceiling: 14336x4096 n = 512 has the VALU busy 53% of the time and the matrix cores 19%, and its
+// waves wait for a stage's copies or the barrier 21% of theirs (grouped: 43%, 15%, 37%). With the prep, f16 kernel -> this one: 14336x4096 n = 512 103 -> 73 us, n = 2048 373 -> 240 us; the two
 // grouped products of a 32-expert 2 x 5760 / 2880 block at 512 tokens, top-4, 166 + 94 -> 117 + 72 us (of a wave's
 // cycles there 37% wait on copies and barriers, its weights being read once at 3.2 TB/s).
 //
@@ -47,13 +51,6 @@ template <int RT> struct Stage {
     static constexpr int A = 0, H = A + WAVES * RT * 2048, B16 = H + WAVES * 256, B8 = B16 + 8192, DX = B8 + 4096,
                          BYTES = DX + 1024;
 };
-
-template <int I, int N, typename F> JAMHIP_DEV void static_for(const F& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
 
 JAMHIP_DEV void copy16(const void* g, void* l) { __builtin_amdgcn_global_load_lds(g, (lds_void*) l, 16, 0, 0); }
 JAMHIP_DEV void copy4(const void* g, void* l) { __builtin_amdgcn_global_load_lds(g, (lds_void*) l, 4, 0, 0); }
@@ -194,7 +191,7 @@ __global__ void __launch_bounds__(64 * mx4::WAVES, 2) mx4_gemm_kernel(WeightView
                 }
             };
             mul(std::integral_constant<int, 0>{});
-            static_for<0, 4 * NSTEP>([&](auto T) {
+            unroll<0, 4 * NSTEP>([&](auto T) {
                 if constexpr (decltype(T)::value + 1 < 4 * NSTEP) mul(std::integral_constant<int, decltype(T)::value + 1>{});
                 add(T);
             });

@@ -57,8 +57,8 @@ __global__ void __launch_bounds__(256) quant_f2_kernel(const float* __restrict__
 // |d_b| < 2^(F - 39), F the largest fp16 exponent field), or that holds a non-finite
 // scale (MXFP4 e = 255, which jam decodes as +Inf; an fp16 Inf/NaN), sets *flag: the host then keeps the
 // tensor off the matrix cores, on kernels that apply every block scale in f32 as jam does. MXFP4's kernel (mx4.hip) needs
-// e <= MX4_MAX_E alone; tensors with blocks 15 or more binades below their group's largest stay on the other kernels
-// too, which take them as before.
+// e <= MX4_MAX_E alone; tensors with blocks 15 or more binades below their group's largest, which it could take as well, are
+// kept off it only so that what they compute stays what it was (no quantizer output comes near that spread).
 template <int DT>
 __global__ void __launch_bounds__(256) repack_kernel(const uint8_t* __restrict__ raw, int64_t raw_stride,
                                                      int64_t rows, int64_t rb, int64_t G, uint8_t* __restrict__ qs,
@@ -142,16 +142,15 @@ __global__ void __launch_bounds__(256) repack_kernel(const uint8_t* __restrict__
             }
         }
         bool bad = false;   // the matrix cores' folding would not be exact for this row's group
-        if constexpr (DT == MXFP4) {   // byte 8: the largest exponent of the counted blocks; 9..15 zero
-            uint8_t er = 0;
+        if constexpr (DT == MXFP4) {   // bytes 8..15 zero
+            uint8_t er = 0;            // the largest exponent of the counted blocks
             for (int j = 0; j < BPG; j++) {
                 if (!nz[j] && ds[j] != 255) ds[j] = 0;
                 er = ds[j] > er ? ds[j] : er;
                 bad |= ds[j] == 255;
             }
             for (int j = 0; j < BPG; j++) bad |= nz[j] && ((int) ds[j] + 14 < (int) er || ds[j] > MX4_MAX_E);
-            ds[8] = er;
-            for (int t = 9; t < 16; t++) ds[t] = 0;
+            for (int t = 8; t < 16; t++) ds[t] = 0;
         } else {
             uint32_t hs[BPG];
             int F = 0;   // largest fp16 exponent field of the group

@@ -1,26 +1,27 @@
-"""CPU model of the matrix-core GEMM's block-scale folding (Q8_0, Q4_0, MXFP4) and of the repack's guard.
+"""CPU model of the matrix-core GEMMs' block scales (Q8_0, Q4_0, MXFP4) and of the repack's guard.
 
-The matrix-core kernel (qxotic_amd/csrc/mma.hip, kq_gemm_kernel) folds every 32-element block's scale into
-an f16 weight operand relative to a per-row, per-group reference:
-  MXFP4  operand = e2m1(code) * 2^(e_b - e_ref + 1)        (hardware conversion to f16), then 2^(e_ref-128)
+Q8_0 and Q4_0 (qxotic_amd/csrc/mma.hip, kq_gemm_kernel): every 32-element block's scale is folded into an f16 weight
+operand relative to a per-row, per-group reference:
   Q8_0   operand = q * d'_b,   d'_b = f16(d_b * 2^s_r), s_r = 22 - F   (hi + lo f16 split of the product)
   Q4_0   operand = nib * d'_b, d'_b = f16(d_b * 2^s_r), s_r = 25 - F   (F: largest fp16 exponent field)
-and applies jam's per-block activation scale dx_b with one f32 FMA per block. This file restates that
-arithmetic in numpy (float16 rounds to nearest even like the hardware conversions; a second model also
-flushes f16 subnormals to zero) and checks it against the oracle's jam F2 result (jo_mm_int8 flavour 2,
-libjam-pinned in test_oracle.py) under the tier-1 bound.
+MXFP4 (qxotic_amd/csrc/mx4.hip): one scaled product per block holds the fp4 codes against the sign and the two digits of each
+activation code, |q| = 16h + l, in fp6: e2m1(code)·(h / 8)·2^7 + e2m1(code)·(l / 8)·2^3, times 2^(e - 127), in f32.
+Each applies jam's per-block activation scale dx_b with one f32 FMA per block. This file restates that arithmetic in numpy
+(float16 rounds to nearest even like the hardware conversions; a second model also flushes f16 subnormals to zero) and
+checks it against the oracle's jam F2 result (jo_mm_int8 flavour 2, libjam-pinned in test_oracle.py) under the tier-1 bound.
 
-It shows the cases the earlier reference rule (e_ref / F over every block of the group) got wrong, and that
-under the repack's rule (qxotic_amd/csrc/prep.hip, repack_kernel: blocks with all-zero products do not set
-the reference; groups spanning more than the f16 range, or holding a non-finite scale, are flagged and
-kept off the matrix cores) every group that is not flagged folds exactly: each operand equals its exact
-value in both models.
+It shows the cases the earlier reference rule of Q8_0 and Q4_0 (F over every block of the group) got wrong, and that under the
+repack's rule (qxotic_amd/csrc/prep.hip, repack_kernel: blocks with all-zero products do not set the reference; groups
+spanning more than the f16 range, MXFP4 exponents past 238, or a non-finite scale, are flagged and kept off the matrix
+cores) every group that is not flagged is exact before its FMA: each folded operand, or MXFP4's whole block sum, equals its
+exact value.
 """
 import numpy as np
 import pytest
 
 from oracle import oracle as O
 
+MX4_MAX_E = 238   # common.h
 KV = np.array([0, 1, 2, 3, 4, 6, 8, 12, 0, -1, -2, -3, -4, -6, -8, -12], np.int64)   # e2m1 value x 2
 
 
@@ -68,16 +69,14 @@ def decode_group(dt, row):
 
 # ------------------------------------------------------------------------------ the repack's rule
 def guard(dt, scale, codes, nib, rule):
-    """(stored scales, reference, flagged) of one group. rule 'old': the reference from every block, nothing
-    flagged; 'new': repack_kernel's rule."""
+    """(stored scales, reference, flagged) of one group. rule 'old' (Q8_0, Q4_0): the reference from every block,
+    nothing flagged; 'new': repack_kernel's rule."""
     scale = scale.copy()
     if dt == O.MXFP4:
-        if rule == "old":
-            return scale, int(scale.max()), False
         nz = ((nib & 7) != 0).any(axis=1)
         scale[~nz & (scale != 255)] = 0
         er = int(scale.max())
-        bad = bool((scale == 255).any() or (nz & (scale + 14 < er)).any())
+        bad = bool((scale == 255).any() or (nz & ((scale + 14 < er) | (scale > MX4_MAX_E))).any())
         return scale, er, bad
     if rule == "new" and dt == O.Q8_0:
         nz = (codes != 0).any(axis=1)
@@ -93,14 +92,8 @@ def guard(dt, scale, codes, nib, rule):
 
 
 def operands(dt, scale, codes, ref, flush):
-    """The kernel's folded f16 weight operands [8, 32] (Q8_0 / Q4_0: hi + lo) and the row factor that undoes
-    the folding at the group end; and the exact values they stand for."""
-    if dt == O.MXFP4:
-        ex = scale - ref + 128
-        fac = np.where(ex > 0, np.exp2((ex - 127).astype(np.float64)), 0.0)
-        w16 = as_f16((codes / 2.0) * fac[:, None], flush)
-        exact = (codes / 2.0) * np.exp2((scale - ref + 1).astype(np.float64))[:, None]
-        return w16, exact, 2.0 ** (ref - 128)
+    """The kernel's folded f16 weight operands [8, 32] (hi + lo) and the row factor that undoes the folding at the
+    group end; and the exact values they stand for."""
     s_r = (22 if dt == O.Q8_0 else 25) - ref
     d = f16_of(scale)
     dh = as_f16(d * 2.0 ** s_r, flush)
@@ -109,13 +102,33 @@ def operands(dt, scale, codes, ref, flush):
     return hi + lo, codes * (d * 2.0 ** s_r)[:, None], 2.0 ** -s_r
 
 
+E2M1 = KV / 2.0                                                                    # fp4 codes
+E2M3 = np.array([m / 8 if e == 0 else (1 + m / 8) * 2.0 ** (e - 1) for e in range(4) for m in range(8)])   # fp6, sign bit apart
+
+
+def mx4_blocks(scale, nib, xq):
+    """The scaled product of each block [8] for activation codes [256], exactly, from the operands' own decodings."""
+    q = xq.reshape(8, 32).astype(np.int64)
+    sign, mag = np.where(q < 0, -1.0, 1.0), np.abs(q)
+    hi, lo = sign * E2M3[mag >> 4] * 2.0 ** 7, sign * E2M3[mag & 15] * 2.0 ** 3
+    return (E2M1[nib] * (hi + lo)).sum(1) * np.exp2(scale.astype(np.float64) - 127)
+
+
 def kernel_row(dt, row, xq, dx, xs, rule, flush):
     """One weight row of k = 256 (one group) against F2 activations [n]: the kernel's arithmetic."""
     scale, codes, nib = decode_group(dt, row)
     sc, ref, _ = guard(dt, scale, codes, nib, rule)
-    w, _, fac = operands(dt, sc, codes, ref, flush)
     n = xq.shape[0]
     out = np.zeros(n, np.float32)
+    if dt == O.MXFP4:
+        for j in range(n):
+            P = mx4_blocks(sc, nib, xq[j]).astype(np.float32)
+            accs = np.float32(float(P[0]) * float(dx[j, 0]))
+            for b in range(1, 8):
+                accs = np.float32(float(P[b]) * float(dx[j, b]) + float(accs))   # f32 fma
+            out[j] = accs
+        return out
+    w, _, fac = operands(dt, sc, codes, ref, flush)
     for j in range(n):
         accs = np.float32(0.0)
         for b in range(8):
@@ -168,6 +181,8 @@ def mx_cases():
         cases[f"spread {s}, reference block's activations zero"] = (np.concatenate(blocks), (0,))
     cases["all e=0"] = (np.concatenate([mx_block(0, rand_nibs(rng)) for _ in range(8)]), ())
     cases["e=0 beside e=1..3"] = (np.concatenate([mx_block(b % 4, rand_nibs(rng)) for b in range(8)]), ())
+    for top in (238, 239, 254):
+        cases[f"all e={top}"] = (np.concatenate([mx_block(top, rand_nibs(rng)) for _ in range(8)]), ())
     cases["e=255 block"] = (np.concatenate([mx_block(255, rand_nibs(rng))] + normal[1:]), ())
     return cases
 
@@ -193,12 +208,44 @@ def q_cases(dt):
     return cases
 
 
-@pytest.mark.parametrize("dt", [O.MXFP4, O.Q8_0, O.Q4_0])
+def test_mx4_code_digits():
+    """Every activation code splits into a sign and two digits that fp6 e2m3 holds as integers over 8, and the two scaled
+    digits add up to the code; the largest block sum under the largest accepted exponent is finite and exact in f32."""
+    q = np.arange(-128, 128)
+    mag = np.abs(q)
+    assert (E2M3[mag >> 4] * 8 == mag >> 4).all() and (E2M3[mag & 15] * 8 == (mag & 15)).all()
+    assert (np.sign(q) * (E2M3[mag >> 4] * 2.0 ** 7 + E2M3[mag & 15] * 2.0 ** 3) == q).all()
+    for e in (0, 1, 127, MX4_MAX_E):
+        for code, x in ((7, 127), (7, -128), (15, -128), (1, 1)):
+            P = mx4_blocks(np.full(8, e), np.full((8, 32), code), np.full(256, x))
+            assert (P == 32 * KV[code] * x * 2.0 ** (e - 128)).all()
+            assert np.isfinite(P.astype(np.float32)).all() and (P.astype(np.float32) == P).all()
+
+
+@pytest.mark.parametrize("case", list(mx_cases()))
+def test_mx4_edge_cases(oracle, case):
+    """Every edge case is either flagged (kept off the matrix cores) or meets the tier-1 bound with exact f32 block sums."""
+    row, zb = mx_cases()[case]
+    scale, codes, nib = decode_group(O.MXFP4, row)
+    sc, _, flagged = guard(O.MXFP4, scale, codes, nib, "new")
+    spread = int(case.split()[1].rstrip(",")) if case.startswith("spread") else 0
+    assert flagged == (spread > 14 or "255" in case or "all e=239" in case or "all e=254" in case)
+    if flagged:
+        return
+    a = activations(oracle, 300, zb) * np.float32(2.0 ** -100 if "238" in case else 1.0)
+    xq, _, _ = oracle.quant_f2(a)
+    for j in range(a.shape[0]):
+        P = mx4_blocks(sc, nib, xq[j])
+        assert (P.astype(np.float32) == P).all()
+    assert run_case(oracle, O.MXFP4, row, a, "new", False)
+
+
+@pytest.mark.parametrize("dt", [O.Q8_0, O.Q4_0])
 def test_edge_cases_old_rule_vs_repack_rule(oracle, dt):
     """Every edge case: under the repack's rule the group is either flagged (kept off the matrix cores) or
     folds to the tier-1 answer in both f16 models. The earlier rule's failures are listed and asserted, so
     the finding stays on record."""
-    cases = mx_cases() if dt == O.MXFP4 else q_cases(dt)
+    cases = q_cases(dt)
     old_fail, report = [], []
     for i, (name, (row, zb)) in enumerate(cases.items()):
         a = activations(oracle, 100 + i, zb)
@@ -213,9 +260,6 @@ def test_edge_cases_old_rule_vs_repack_rule(oracle, dt):
         report.append(f"{name}: old {'ok' if ok_old else 'FAILS tier 1'}, new {'flagged' if flagged else 'exact'}")
     print(f"\n{O.NAMES[dt]}:\n  " + "\n  ".join(report))
     expect_old_fail = {
-        O.MXFP4: {"e254 zero-code block beside e~120", "e254 -0-code block beside e~120",
-                  "spread 15, reference block's activations zero", "spread 20, reference block's activations zero",
-                  "spread 30, reference block's activations zero", "spread 60, reference block's activations zero"},
         O.Q8_0: {"fp16-max scale on a zero-code block", "spread 2^22, reference block's activations zero",
                  "spread 2^24, reference block's activations zero", "spread 2^25, reference block's activations zero",
                  "spread 2^30, reference block's activations zero"},
@@ -228,9 +272,8 @@ def test_edge_cases_old_rule_vs_repack_rule(oracle, dt):
 def test_unflagged_groups_fold_exactly(dt):
     """2000 random groups with block scales spread over up to 40 binades (fp16 scales from 2^14 down, into
     the subnormals and to zero) and random all-zero blocks: every group the repack's rule does not flag has
-    every folded f16 operand equal to its exact value. MXFP4's operands are normal f16 values, so this holds
-    with and without subnormals; Q8_0 / Q4_0 keep d'_b normal, but the lo part of a product's hi + lo split
-    can be an f16 subnormal, which the device keeps (test_gpu_fold.py checks the accepted limit at the
+    every folded f16 operand, or MXFP4's block sum of random codes in f32, equal to its exact value. Q8_0 / Q4_0 keep
+    d'_b normal, but the lo part of a product's hi + lo split can be an f16 subnormal, which the device keeps (test_gpu_fold.py checks the accepted limit at the
     error floor, where a flushed lo part would show). Flagging is not over-eager: spreads inside the f16
     range are never flagged."""
     rng = np.random.default_rng(0xF01D ^ dt)
@@ -259,7 +302,12 @@ def test_unflagged_groups_fold_exactly(dt):
             assert spread > lim, (spread, O.NAMES[dt])
             continue
         seen["exact"] += 1
-        for flush in ((False, True) if dt == O.MXFP4 else (False,)):
-            w, exact, _ = operands(dt, sc, codes, ref, flush)
-            assert np.array_equal(w, exact), (O.NAMES[dt], spread, flush)
+        if dt == O.MXFP4:
+            xq = rng.integers(-128, 128, 256)
+            P = mx4_blocks(sc, nib, xq)
+            exact = (codes * xq.reshape(8, 32)).sum(1) * np.exp2(sc.astype(np.float64) - 128)
+            assert (P == exact).all() and (P.astype(np.float32) == P).all()
+            continue
+        w, exact, _ = operands(dt, sc, codes, ref, False)
+        assert np.array_equal(w, exact), (O.NAMES[dt], spread)
     assert seen["flagged"] > 100 and seen["exact"] > 500, seen
